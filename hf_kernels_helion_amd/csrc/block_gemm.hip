@@ -1455,16 +1455,28 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
 // split-K path). Waves of WM x WN (two per SIMD for 64x32); with half the operand
 // reuse of a 256x256 tile this size is bound by the operand stream, so it
 // keeps three K-blocks of DMA in flight: four LDS stages of 32 KiB, the DMA
-// of K-block kb+4 issued right after the barrier that opens K-block kb. Each
-// K-block's fragments are read from LDS during the previous K-block's MFMAs
-// into the other of two register sets; scale windows and asm DMA as in
-// gemm_pipe256_kernel.
+// of K-block kb+4 issued between the MFMAs of K-block kb, after the barrier
+// that opens it. Each K-block's fragments are read from LDS during the
+// previous K-block's MFMAs into the other of two register sets; scale windows
+// and asm DMA as in gemm_pipe256_kernel.
+// What bounds it: per K-block and CU the MFMAs and folds alone take 0.30 us,
+// the LDS reads alone 0.23, the DMA alone 0.36 (timing-only builds at
+// 1000x4096x7168), and together 0.52: LDS reads and DMA writes share the LDS
+// while two waves per SIMD share the matrix core. 0.63 before the K-block
+// body was free of branches (2048x2048x4096 25.1 -> 20.9 us, 1000x4096x7168
+// with fp32 output 42.0 -> 35.2). Measured slower: four waves of 64x64 (two
+// thirds of the LDS reads, but one wave per SIMD: 28.5 against 23.2 us at
+// 2048x2048x4096), all DMA of a K-block right after its barrier (2%), the
+// scales read before the fragments (2%); level within 0.5%: DMA after odd
+// MFMAs, a raised wave priority over the first MFMAs.
 // ---------------------------------------------------------------------------
 template <int WM, int WN, bool PR>
 __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_kernel(GemmArgs a) {
   constexpr int BM = 128, BN = 128, NWN = BN / WN, NW = (BM / WM) * NWN;
   constexpr int FM = WM / 16, FN = WN / 16;
   static_assert(FM * FN >= FM + FN + 1, "next-K-block reads must fit between the MFMAs");
+  constexpr int SCALE_P = 5;               // MFMA after which the next K-block's scales are read
+  static_assert(SCALE_P >= 2 && FM * FN >= 2 * (BM + BN) / 8 / NW, "see the K-block body");
   static_assert(NW >= BM / 32, "one scale-window instruction per 32 activation rows");
   constexpr int NSTAGE = 4;
   constexpr int STAGE = (BM + BN) * 128;   // 32 KiB
@@ -1476,7 +1488,9 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
   constexpr int EPI_PITCH = WN * 2 + 16;
   constexpr int EPI = NW * WM * EPI_PITCH;
   constexpr int SMEM = (SW_OFF + 2 * WIN > EPI) ? SW_OFF + 2 * WIN : EPI;
-  constexpr int LPW = (BM + BN) / 8 / NW;  // wave-loads per wave per K-block (8)
+  constexpr int LPW = (BM + BN) / 8 / NW;  // wave-loads per wave per K-block (4)
+  constexpr int A_LOADS = BM / 8 / NW;     // wave-loads i < A_LOADS bring A rows
+  static_assert((BM / 8) % NW == 0, "a wave-load is all A or all B rows");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[SMEM];
 
   const int tid = threadIdx.x;
@@ -1511,11 +1525,10 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
   auto issue_op = [&](int kb, int stage, int i) {
     const int L = wid + i * NW;
     const uint32_t lds = lds0 + stage * STAGE + L * 1024;
-    const bool is_a = L < BM / 8;
-    const int Lr = is_a ? L : L - BM / 8;
+    const int Lr = i < A_LOADS ? L : L - BM / 8;
     const int row = (Lr >> 3) * 64 + r8 * 8 + (Lr & 7);
     const int c16 = ((lane & 7) ^ (Lr & 7)) * 16;
-    if (is_a) {
+    if (i < A_LOADS) {
       const uint32_t voff = (uint32_t)min(row, a_lim) * (uint32_t)a.lda + c16;
       dma16_soff(voff, a_base + (int64_t)kb * 128, lds);
     } else {
@@ -1564,7 +1577,7 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
     const int rel = kb - kb_begin;
     if ((rel & 7) == 0) issue_win(kb, (rel >> 3) & 1);
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) issue_op(kb, rel % NSTAGE, i);
+    for (int i = 0; i < LPW; ++i) issue_op(kb, rel & (NSTAGE - 1), i);
   };
 
   const int r7 = lane & 7, g2 = 2 * (lane >> 4);
@@ -1581,7 +1594,7 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
   v8i xf[2][FM], wf[2][FN];
-  float sc[2][FM];
+  float sc[2][FM], sa_n[FM], sb_n = 1.f;  // sa_n, sb_n: the next K-block's, as read
   v4f sbr[2][PR ? FN : 1];  // PR: the weight-row scales of the lane's 4 columns
   v4f r1 = v4f{0.f, 0.f, 0.f, 0.f}, r2 = r1;
   // Scale of output (row i, column group j, element e) in register set S.
@@ -1590,31 +1603,39 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
     else return sc[S][i];
   };
 
-  // Fragments and scales of K-block kb into register set S (reads spread
-  // over the caller's MFMAs by the caller's sched barriers).
-  auto read_frag = [&](int kb, int S, int f) {
-    const uint8_t* st = smem + ((kb - kb_begin) % NSTAGE) * STAGE;
-    if (f < FM) xf[S][f] = lds_frag2(st + q_off + frag_off(wm * FM + f), slo, shi);
-    else wf[S][f - FM] = lds_frag2(st + BM * 128 + q_off + frag_off(wn * FN + f - FM), slo, shi);
+  // Fragment f of a wave's rows starts at the wave's first fragment plus an
+  // offset that does not depend on the wave, so one address register per
+  // operand and 16-byte half serves every read of a K-block.
+  static_assert((4 % FM == 0 || FM % 4 == 0) && (4 % FN == 0 || FN % 4 == 0),
+                "a wave's fragments stay within whole groups of four");
+  const uint8_t* a_frag = smem + q_off + frag_off(wm * FM);
+  const uint8_t* b_frag = smem + BM * 128 + q_off + frag_off(wn * FN);
+  // Fragments and scales of the K-block at LDS offset st (its stage) into
+  // register set S (reads spread over the caller's MFMAs by the caller's
+  // sched barriers).
+  auto read_frag = [&](int st, int S, int f) {
+    if (f < FM) xf[S][f] = lds_frag2(a_frag + st + frag_off(f), slo, shi);
+    else wf[S][f - FM] = lds_frag2(b_frag + st + frag_off(f - FM), slo, shi);
   };
   auto read_scales = [&](int kb, int S) {
     const int rel = kb - kb_begin;
     const int o = ((rel >> 3) & 1) * WIN + (rel & 7) * 4;
-    if constexpr (PR) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-        sc[S][i] = *reinterpret_cast<const float*>(smem + sa_off + o + i * 512);
+    for (int i = 0; i < FM; ++i)
+      sa_n[i] = *reinterpret_cast<const float*>(smem + sa_off + o + i * 512);
+    if constexpr (PR) {
       const int ob = ((rel >> 3) & 1) * WIN + (rel & 7) * 512;
 #pragma unroll
       for (int j = 0; j < FN; ++j)
         sbr[S][j] = *reinterpret_cast<const v4f*>(
             smem + sb_off + ob + (wn * WN + j * 16 + 4 * (lane >> 4)) * 4);
     } else {
-      const float sb = *reinterpret_cast<const float*>(smem + sb_off + o);
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-        sc[S][i] = *reinterpret_cast<const float*>(smem + sa_off + o + i * 512) * sb;
+      sb_n = *reinterpret_cast<const float*>(smem + sb_off + o);
     }
+  };
+  auto set_scales = [&](int S) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i) sc[S][i] = PR ? sa_n[i] : sa_n[i] * sb_n;
   };
 
   // Waits until this wave's DMA of a K-block has landed, given how many
@@ -1632,20 +1653,33 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
     wait_after(min(NSTAGE, nkb) - 1);
     __syncthreads();
 #pragma unroll
-    for (int f = 0; f < FM + FN; ++f) read_frag(kb_begin, 0, f);
+    for (int f = 0; f < FM + FN; ++f) read_frag(0, 0, f);
     read_scales(kb_begin, 0);
+    set_scales(0);
   }
 
-  auto body = [&](int kb, auto set_tag) {
+  // One K-block. KIND 0: steady state (the next K-block is there, and so is
+  // kb + NSTAGE to fetch); 1: the next K-block is there, kb + NSTAGE perhaps;
+  // 2: the last K-block. A KIND known at compile time keeps the body free of
+  // branches: with run-time tests around the reads the compiler no longer
+  // knows how many are in flight and waits for all of them (lgkmcnt(0)) in
+  // the middle of the MFMAs.
+  auto body = [&](int kb, auto set_tag, auto kind_tag) {
     constexpr int S = decltype(set_tag)::value, T = S ^ 1;
-    const bool more = kb + 1 < kb_end;
-    if (more) {
+    constexpr int KIND = decltype(kind_tag)::value;
+    const int nst = ((kb + 1 - kb_begin) & (NSTAGE - 1)) * STAGE;
+    if constexpr (KIND < 2) {
       // outstanding: the DMAs of kb+1 .. min(kb+3, kb_end-1)
-      wait_after(min(2, kb_end - kb - 2));
+      if constexpr (KIND == 0) wait_vmcnt<2 * LPW>();
+      else wait_after(min(2, kb_end - kb - 2));
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();
-      if (kb + NSTAGE < kb_end) issue_kb(kb + NSTAGE);
     }
+    // DMA of kb + NSTAGE into the stage this K-block's fragments have left,
+    // one instruction after every other MFMA
+    const bool fill = KIND == 0 || (KIND == 1 && kb + NSTAGE < kb_end);
+    const int rel_n = kb + NSTAGE - kb_begin;
+    if (fill && (rel_n & 7) == 0) issue_win(kb + NSTAGE, (rel_n >> 3) & 1);
 #pragma unroll
     for (int p = 0; p < FM * FN; ++p) {
       const int i = p / FN, j = p % FN;
@@ -1666,9 +1700,14 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
       }
       r2 = r1;
       r1 = res;
-      if (more) {
-        if (p < FM + FN) read_frag(kb + 1, T, p);
-        if (p == FM + FN) read_scales(kb + 1, T);
+      if constexpr (KIND < 2) {
+        if (fill && (p & 1) == 0 && p / 2 < LPW)
+          issue_op(kb + NSTAGE, rel_n & (NSTAGE - 1), p / 2);
+        if (p < FM + FN) read_frag(nst, T, p);
+        // (set T still holds the previous K-block's scales for its last two
+        // folds, at MFMAs 0 and 1)
+        if (p == SCALE_P) read_scales(kb + 1, T);
+        if (p == FM * FN - 1) set_scales(T);
       }
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
@@ -1680,14 +1719,24 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
   for (int i = 0; i < FM; ++i) sc[1][i] = 0.f;
 #pragma unroll
   for (int j = 0; j < (PR ? FN : 1); ++j) sbr[1][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  using K0 = PipeKind<0>;
+  using K1 = PipeKind<1>;
+  using K2 = PipeKind<2>;
   int kb = kb_begin;
-  for (; kb + 1 < kb_end; kb += 2) {
-    body(kb, PipeKind<0>{});
-    body(kb + 1, PipeKind<1>{});
+  for (; kb + 1 + NSTAGE < kb_end; kb += 2) {
+    body(kb, K0{}, K0{});
+    body(kb + 1, K1{}, K0{});
+  }
+  for (; kb + 2 < kb_end; kb += 2) {
+    body(kb, K0{}, K1{});
+    body(kb + 1, K1{}, K1{});
   }
   int last_set = 1;
-  if (kb < kb_end) {
-    body(kb, PipeKind<0>{});
+  if (kb + 1 < kb_end) {
+    body(kb, K0{}, K1{});
+    body(kb + 1, K1{}, K2{});
+  } else if (kb < kb_end) {
+    body(kb, K0{}, K2{});
     last_set = 0;
   }
   if (nkb > 0) {
