@@ -23,9 +23,9 @@
 //   * Split-K writes fp32 partials to the caller's workspace; a second kernel
 //     sums them in split order and applies the output conversion.
 //
-// Generic path (any block_n/block_k, ragged K, unaligned operands): a SIMT
-// kernel with the same blockwise summation, used only where the MFMA path's
-// preconditions do not hold.
+// Generic path (any block_n/block_k, ragged K, unaligned operands): fp16 MFMAs
+// on converted codes with the same blockwise summation, used only where the
+// fp8 MFMA path's preconditions do not hold.
 #include "common.h"
 #include "quant.h"
 
@@ -2844,9 +2844,41 @@ splitk_reduce_xcd_kernel(GemmArgs a, int splits) {
   store4(a, m, n, s, false, 0);
 }
 
-// Generic SIMT kernel: 32x32 outputs per 256-thread block, 2x2 per thread.
-// For each K-block: part = sum_k A*B over the block (fp32 FMA chain in k
-// order), then acc += part * As * Bs, as in fp8.py:31-37.
+// ---------------------------------------------------------------------------
+// Generic kernel: any block_n, block_k, K, alignment and strides (ragged K,
+// block sizes other than 128, unaligned rows, leading dimensions past 32-bit
+// offsets). For each K-block: part = sum_k A*B over the block, then
+// acc += part * As * Bs, as in fp8.py:31-37.
+//
+// The sums keep fp32 precision, which the fp8 MFMA's (truncated to about
+// 2^-13 of the largest product) do not: the codes are converted to fp16,
+// which holds every e4m3fn value exactly, and multiplied by
+// v_mfma_f32_16x16x32_f16, whose products of two such values are exact and
+// whose fp32 sums measured closer to 64 bits than a chain of 128 fp32 FMAs
+// (relative 2-norm 7.9e-8 against 1.3e-7 on codes spread over the format's
+// range, 9.4e-9 against 1.0e-8 on normal ones).
+//
+// K is walked in chunks of 128 bytes that never cross a K-block, zero past
+// its end, and each chunk's sum is folded by itself (a K-block longer than 128
+// with the same scales for each of its chunks). A wave owns 16*FM activation rows x 16*FN weight rows. The rows of
+// a chunk go through registers into LDS (eight lanes of 16 bytes per row, at
+// any alignment; the next chunk and its scales are in flight while this one
+// is multiplied),
+// 16-byte piece c of row R in slot c ^ (R/2 % 8), so that the fragment reads
+// (16 rows, one piece) meet distinct banks; fragments are converted after the
+// read. Lane l holds bytes 32*(l/16)..+31 of row l%16 of a fragment, and step
+// s of a chunk multiplies bytes 8s..8s+7 of every lane, the same K for both
+// operands. KW = 1: four waves on 2 x 2 tiles share two LDS buffers, one
+// barrier per chunk. KW > 1 (few rows or few tiles): each wave stages its own
+// rows, without barriers, the waves split the K-blocks of one tile and sum
+// through LDS in wave order.
+// Bound: converts, folds and MFMAs of two waves per SIMD, which overlap only
+// in part (0.85 us per 64x128 tile and chunk and CU, 0.21 of it MFMAs):
+// 4096x4096x4080 213 us (645 TFLOP/s), 777x4096x1376 22.8 us against 330 on
+// the SIMT kernel this replaces. Measured slower: fragments straight from
+// global memory without LDS (43.5 us at 777x4096x1376: four cache lines per
+// four lanes), loads two chunks ahead (25.5 us), 128x128 tiles (46.7).
+// ---------------------------------------------------------------------------
 struct GenericArgs {
   const uint8_t* A;
   const uint8_t* B;
@@ -2855,66 +2887,293 @@ struct GenericArgs {
   void* C;
   int64_t lda, ldb, as_sm, as_sk, bs_sn, bs_sk, ldc;
   int64_t M, N, K, block_n, block_k;
+  int64_t KB;     // K-blocks: ceil(K / block_k)
   int out_dtype;
+  int vec_store;  // four consecutive outputs can be stored as one vector
 };
 
-__global__ void __launch_bounds__(256) gemm_generic_kernel(GenericArgs g) {
-  __shared__ float sA[32][33];
-  __shared__ float sB[32][33];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int64_t mb = (int64_t)blockIdx.y * 32, nbase = (int64_t)blockIdx.x * 32;
-  float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-  const int64_t KB = (g.K + g.block_k - 1) / g.block_k;
-  for (int64_t kb = 0; kb < KB; ++kb) {
-    float part[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-    const int64_t kbeg = kb * g.block_k, kend = min(kbeg + g.block_k, g.K);
-    for (int64_t k0 = kbeg; k0 < kend; k0 += 32) {
-      for (int e = threadIdx.x; e < 32 * 32; e += 256) {
-        const int r = e >> 5, c = e & 31;
-        const int64_t k = k0 + c;
-        const int64_t m = mb + r, n = nbase + r;
-        sA[r][c] = (m < g.M && k < kend) ? fp8e4m3_to_f32(g.A[m * g.lda + k]) : 0.f;
-        sB[r][c] = (n < g.N && k < kend) ? fp8e4m3_to_f32(g.B[n * g.ldb + k]) : 0.f;
-      }
-      __syncthreads();
-      for (int c = 0; c < 32; ++c) {
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
+// 8 e4m3fn codes as fp16 (every code is exact, NaN stays NaN).
+__device__ __forceinline__ h8 fp8x8_to_f16(uint32_t lo, uint32_t hi) {
+  const h2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, false);
+  const h2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, true);
+  const h2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, false);
+  const h2 d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, true);
+  return h8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+// 16 bytes at any alignment (global loads need none on this target).
+__device__ __forceinline__ v4i load16_any(const uint8_t* p) {
+  v4i v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+// v without its first `skip` bytes, the following `valid` (0..16) bytes kept
+// and zeros after them.
+__device__ __forceinline__ v4i keep_bytes(const v4i v, int skip, int valid) {
+  uint64_t lo = (uint32_t)v[0] | ((uint64_t)(uint32_t)v[1] << 32);
+  uint64_t hi = (uint32_t)v[2] | ((uint64_t)(uint32_t)v[3] << 32);
+  if (skip >= 8) {
+    lo = hi >> (8 * (skip & 7));
+    hi = 0;
+  } else if (skip > 0) {
+    lo = (lo >> (8 * skip)) | (hi << (64 - 8 * skip));
+    hi >>= 8 * skip;
+  }
+  if (valid < 8) {
+    lo = valid <= 0 ? 0 : lo & ((uint64_t(1) << (8 * valid)) - 1);
+    hi = 0;
+  } else if (valid < 16) {
+    hi &= (uint64_t(1) << (8 * (valid - 8))) - 1;
+  }
+  return v4i{(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi,
+             (int)(uint32_t)(hi >> 32)};
+}
+
+// `n` (0..15) bytes at p one by one, zeros after them.
+__device__ __forceinline__ v4i load_bytes(const uint8_t* p, int n) {
+  uint64_t lo = 0, hi = 0;
+#pragma unroll 1
+  for (int b = n - 1; b >= 0; --b) {
+    hi = (hi << 8) | (lo >> 56);
+    lo = (lo << 8) | p[b];
+  }
+  return v4i{(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi,
+             (int)(uint32_t)(hi >> 32)};
+}
+
+// FM x FN fragments per wave. BN16: block_n is a multiple of 16, so a
+// fragment's columns share one weight scale (else one scale per column).
+// SHORT: K < 16, rows read byte by byte.
+template <int FM, int FN, int KW, bool BN16, bool SHORT = false>
+__global__ void __launch_bounds__(KW == 1 ? 256 : 64 * KW, 2) gemm_generic_kernel(GenericArgs g) {
+  constexpr int NWM = KW == 1 ? 2 : 1, NWN = KW == 1 ? 2 : 1;
+  constexpr int NSB = BN16 ? 1 : 4;      // weight scales per lane and fragment
+  constexpr int AR = 16 * NWM * FM;      // activation rows staged together
+  constexpr int ROWS = AR + 16 * NWN * FN;
+  constexpr int SW = KW == 1 ? 4 : 1;    // waves that stage them
+  constexpr int PER = ROWS / 8 / SW;     // 8-row pieces per wave
+  constexpr int BUFS = KW == 1 ? 2 : 1;  // (a wave's own LDS accesses stay in order)
+  static_assert(ROWS % (8 * SW) == 0, "whole pieces per wave");
+  constexpr int STAGE = ROWS * 128, OPS = KW * BUFS * STAGE;
+  constexpr int RED = KW == 1 ? 0 : KW * FM * FN * 64 * 16;
+  __shared__ __attribute__((aligned(256))) uint8_t smem[OPS > RED ? OPS : RED];
+
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = KW == 1 ? wid >> 1 : 0, wn = KW == 1 ? wid & 1 : 0, kw = KW == 1 ? 0 : wid;
+  const int64_t m_wg = (int64_t)blockIdx.y * AR, n_wg = (int64_t)blockIdx.x * (ROWS - AR);
+  const int64_t m0 = m_wg + wm * 16 * FM, n0 = n_wg + wn * 16 * FN;
+  const int r = lane & 15, q = lane >> 4;
+
+  // This wave's K-blocks.
+  const int64_t per = (g.KB + KW - 1) / KW;
+  const int64_t kb_begin = min(kw * per, g.KB);
+  const int64_t kb_end = min(kb_begin + per, g.KB);
+
+  // Rows this lane stages (rows past the edge clamped; their outputs are not
+  // stored), and the scales of the rows and columns it accumulates.
+  const uint8_t* src[PER];
+  int dst[PER];
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < PER; ++i) {
+    const int R = ((KW == 1 ? wid : 0) + i * SW) * 8 + (lane >> 3);
+    src[i] = (R < AR ? g.A + min(m_wg + R, g.M - 1) * g.lda
+                     : g.B + min(n_wg + R - AR, g.N - 1) * g.ldb) + 16 * (lane & 7);
+    dst[i] = R * 128 + (((lane & 7) ^ ((R >> 1) & 7)) << 4);
+  }
+  const float* as_row[FM];
+  const float* bs_row[FN][NSB];
+  auto block_row = [&](int64_t n) -> int64_t {  // 32-bit division where it fits
+    if (g.block_n == 1) return n;
+    if (((g.N | g.block_n) >> 31) == 0) return (uint32_t)n / (uint32_t)g.block_n;
+    return n / g.block_n;
+  };
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
-            part[i][j] = fmaf(sA[ty * 2 + i][c], sB[tx * 2 + j][c], part[i][j]);
-      }
-      __syncthreads();
+  for (int i = 0; i < FM; ++i) as_row[i] = g.As + min(m0 + 16 * i + r, g.M - 1) * g.as_sm;
+#pragma unroll
+  for (int j = 0; j < FN; ++j)
+#pragma unroll
+    for (int e = 0; e < NSB; ++e)
+      bs_row[j][e] =
+          g.Bs + block_row(min(n0 + 16 * j + (BN16 ? 0 : 4 * q + e), g.N - 1)) * g.bs_sn;
+
+  v4f acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  uint8_t* own = smem + kw * STAGE;  // KW > 1: this wave's rows
+  // Rows and scales of the chunk being loaded (past the last chunk it is loaded
+  // again: without a branch around them the compiler knows how many loads are
+  // in flight).
+  v4i st[PER];
+  float sa_n[FM], sb_n[FN][NSB];
+  int64_t k_st = 0, kend_st = 0;
+  int64_t kb_l = kb_begin, k_l = kb_begin * g.block_k, kend_l = min(k_l + g.block_k, g.K);
+  const int c16 = 16 * (lane & 7);
+  // Bytes k..k+127 of the staged rows into registers. A 16-byte piece that
+  // runs past its row's end is read as the row's last 16 bytes (K >= 16), so
+  // no load leaves its row; write() then drops the bytes read too early and
+  // clears those from kend on.
+  auto load = [&]() {
+    k_st = k_l;
+    kend_st = kend_l;
+    if constexpr (SHORT) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        st[i] = load_bytes(src[i] + k_l, (int)max(kend_l - k_l - c16, (int64_t)0));
+    } else {
+      const int64_t at = min(k_l + c16, g.K - 16) - c16;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) st[i] = load16_any(src[i] + at);
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int64_t m = min(mb + ty * 2 + i, g.M - 1);
-      const float sa = g.As[m * g.as_sm + kb * g.as_sk];
+    for (int i = 0; i < FM; ++i) sa_n[i] = as_row[i][kb_l * g.as_sk];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int64_t n = min(nbase + tx * 2 + j, g.N - 1);
-        const float sb = g.Bs[(n / g.block_n) * g.bs_sn + kb * g.bs_sk];
-        acc[i][j] = acc[i][j] + part[i][j] * sa * sb;
-      }
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int e = 0; e < NSB; ++e) sb_n[j][e] = bs_row[j][e][kb_l * g.bs_sk];
+    // the chunk after this one: in this K-block or at the next one's start
+    if (k_l + 128 < kend_l) {
+      k_l += 128;
+    } else if (kb_l + 1 < kb_end) {
+      ++kb_l;
+      k_l = kb_l * g.block_k;
+      kend_l = min(k_l + g.block_k, g.K);
+    }
+  };
+  auto write = [&](int buf) {
+    if (!SHORT && k_st + 128 > kend_st) {
+      const int64_t at = k_st + c16;
+      const int valid = (int)max(min(kend_st - at, (int64_t)16), (int64_t)0);
+      const int skip = valid > 0 ? (int)(at - min(at, g.K - 16)) : 0;  // 0..15
+#pragma unroll
+      for (int i = 0; i < PER; ++i) st[i] = keep_bytes(st[i], skip, valid);
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      *reinterpret_cast<v4i*>(own + buf * STAGE + dst[i]) = st[i];
+    asm volatile("" ::: "memory");
+    if constexpr (KW == 1) __syncthreads();
+  };
+  // Fragment of the 16 rows from R0 (a multiple of 16).
+  auto frag = [&](int buf, int R0) {
+    const uint8_t* p = own + buf * STAGE + (R0 + r) * 128;
+    const int sw = (r >> 1) & 7;
+    return lds_frag2(p, ((2 * q) ^ sw) << 4, ((2 * q + 1) ^ sw) << 4);
+  };
+
+  // One chunk from buffer buf.
+  auto chunk = [&](int buf) {
+    float sa[FM], sb[FN][NSB];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) sa[i] = sa_n[i];
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int e = 0; e < NSB; ++e) sb[j][e] = sb_n[j][e];
+    load();
+    v8i xf[FM], wf[FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) xf[i] = frag(buf, (wm * FM + i) * 16);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) wf[j] = frag(buf, AR + (wn * FN + j) * 16);
+    v4f part[FM][FN];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      h8 x[FM], w[FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+        x[i] = fp8x8_to_f16((uint32_t)xf[i][2 * s], (uint32_t)xf[i][2 * s + 1]);
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        w[j] = fp8x8_to_f16((uint32_t)wf[j][2 * s], (uint32_t)wf[j][2 * s + 1]);
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              w[j], x[i], s == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : part[i][j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[i][j][e] = fmaf(part[i][j][e] * sa[i], sb[j][BN16 ? 0 : e], acc[i][j][e]);
+  };
+
+  if (kb_begin < kb_end) {
+    const int64_t last_k = (kb_end - 1) * g.block_k;
+    int64_t left = (kb_end - kb_begin - 1) * ((g.block_k + 127) / 128) +
+                   (min(last_k + g.block_k, g.K) - last_k + 127) / 128;
+    int buf = 0;
+    load();
+    write(0);
+    while (true) {
+      chunk(buf);
+      if (--left == 0) break;
+      // KW = 1: the other buffer was last read before the previous barrier
+      if constexpr (KW == 1) buf ^= 1;
+      write(buf);
     }
   }
+
+  // Lane: output row r of fragment i, columns 4q..4q+3 of fragment j.
+  auto store = [&](int i, int j, const v4f& v) {
+    const int64_t m = m0 + 16 * i + r, n = n0 + 16 * j + 4 * q;
+    if (m >= g.M || n >= g.N) return;
+    const bool vec = n + 4 <= g.N && g.vec_store;
+    if (g.out_dtype == FP8B_F32) {
+      float* p = reinterpret_cast<float*>(g.C) + m * g.ldc + n;
+      if (vec) *reinterpret_cast<v4f*>(p) = v;
+      else for (int e = 0; e < 4 && n + e < g.N; ++e) p[e] = v[e];
+      return;
+    }
+    const bool bf = g.out_dtype == FP8B_BF16;
+    const v2i w = {(int)(bf ? pack_bf16x2(v[0], v[1]) : pack_f16x2(v[0], v[1])),
+                   (int)(bf ? pack_bf16x2(v[2], v[3]) : pack_f16x2(v[2], v[3]))};
+    uint16_t* p = reinterpret_cast<uint16_t*>(g.C) + m * g.ldc + n;
+    if (vec) {
+      *reinterpret_cast<v2i*>(p) = w;
+    } else {
+      for (int e = 0; e < 4 && n + e < g.N; ++e)
+        p[e] = (uint16_t)((uint32_t)w[e >> 1] >> (16 * (e & 1)));
+    }
+  };
+  if constexpr (KW == 1) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int64_t m = mb + ty * 2 + i;
-    if (m >= g.M) continue;
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int64_t n = nbase + tx * 2 + j;
-      if (n >= g.N) continue;
-      const float v = acc[i][j];
-      if (g.out_dtype == FP8B_F32) {
-        reinterpret_cast<float*>(g.C)[m * g.ldc + n] = v;
-      } else if (g.out_dtype == FP8B_BF16) {
-        reinterpret_cast<uint16_t*>(g.C)[m * g.ldc + n] = f32_to_bf16_bits(v);
-      } else {
-        _Float16 h = (_Float16)v;
-        reinterpret_cast<uint16_t*>(g.C)[m * g.ldc + n] = __builtin_bit_cast(uint16_t, h);
+      for (int j = 0; j < FN; ++j) store(i, j, acc[i][j]);
+  } else {
+    // partial tiles summed in wave order, fragment f by wave f % KW, in 64
+    // bits: each wave has rounded its first product already, so an fp32 sum
+    // would round twice more than one wave's chain of FMAs over the same
+    // K-blocks (737x512x288: 5.2e-8 of the result against 4.7e-8)
+    v4f(*red)[FM * FN][64] = reinterpret_cast<v4f(*)[FM * FN][64]>(smem);
+    __syncthreads();  // the staged rows are dead
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) red[wid][i * FN + j][lane] = acc[i][j];
+    __syncthreads();
+    for (int f = wid; f < FM * FN; f += KW) {
+      double s[4] = {0., 0., 0., 0.};
+#pragma unroll
+      for (int w = 0; w < KW; ++w) {
+        const v4f v = red[w][f][lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += (double)v[e];
       }
+      store(f / FN, f % FN, v4f{(float)s[0], (float)s[1], (float)s[2], (float)s[3]});
     }
   }
 }
@@ -3489,6 +3748,44 @@ void resolve_pipe128(Dispatch& d, int64_t tiles, int tail, int cus) {
   d.tail_grid = 4 * rest;
 }
 
+// gemm_generic_kernel's tile (d.bm x d.bn) and waves. 64x128 tiles (2 x 2 waves
+// of 32x64) once they fill the CUs: 4096x4096x4080 213 us against 238 for
+// 64x64 tiles and 375 for 32x32 ones, 777x4096x1376 (416 tiles) 22.8 against
+// 22.8 and 27.7. Below that 32x32 tiles with two waves along K (200x4096x1376
+// 10.1 us against 12.4 on 64x64 tiles), four where the tiles are at most two
+// per CU (64x4096x1376 6.1 against 7.5, 575x512x560 5.7 against 6.5). Up to 32
+// rows, 16x16 tiles with eight waves while they are at most two per CU
+// (16x4096x1376 4.1 against 5.7 us, 32x2048x1001 4.6 against 6.1), for more
+// columns 16x32 tiles up to 16 rows (8x8192x5000 10.8 against 12.1). K < 16
+// (rows read byte by byte): 32x32 tiles, four waves.
+void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int cus) {
+  auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  auto take = [&](int bm, int bn, int waves) {
+    d.kernel = FP8B_KERNEL_GENERIC;
+    d.bm = bm;
+    d.bn = bn;
+    d.waves = waves;
+    d.grid = tiles(bm, bn);
+  };
+  const int64_t c = cus;
+  if (K < 16) take(32, 32, 4);
+  else if (M <= 32 && tiles(16, 16) <= 2 * c) take(16, 16, 8);
+  else if (M <= 16) take(16, 32, 8);
+  else if (tiles(64, 128) >= c) take(64, 128, 4);
+  else take(32, 32, tiles(32, 32) <= 2 * c ? 4 : 2);
+}
+
+template <bool BN16>
+void launch_generic(const GenericArgs& g, const Dispatch& d, hipStream_t st) {
+  const dim3 grid((unsigned)((g.N + d.bn - 1) / d.bn), (unsigned)((g.M + d.bm - 1) / d.bm));
+  if (g.K < 16) gemm_generic_kernel<2, 2, 4, BN16, true><<<grid, 256, 0, st>>>(g);
+  else if (d.bn == 16) gemm_generic_kernel<1, 1, 8, BN16><<<grid, 512, 0, st>>>(g);
+  else if (d.bm == 16) gemm_generic_kernel<1, 2, 8, BN16><<<grid, 512, 0, st>>>(g);
+  else if (d.bm == 64) gemm_generic_kernel<2, 4, 1, BN16><<<grid, 256, 0, st>>>(g);
+  else if (d.waves == 4) gemm_generic_kernel<2, 2, 4, BN16><<<grid, 256, 0, st>>>(g);
+  else gemm_generic_kernel<2, 2, 2, BN16><<<grid, 128, 0, st>>>(g);
+}
+
 // The launches of one GEMM call (see Dispatch) on a device with `cus` CUs.
 Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int64_t block_k,
                           int cus, const Operands& o) {
@@ -3496,9 +3793,8 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
   const bool per_row = block_n == 1 && block_k == 128;
   d.per_row = per_row;
   if (!o.mfma) {
-    d.bm = d.bn = 32;
-    d.grid = ((N + 31) / 32) * ((M + 31) / 32);
-    return d;  // gemm_generic_kernel
+    resolve_generic(d, M, N, K, cus);
+    return d;
   }
   const int KB = (int)(K / 128);
   Plan p = make_plan(M, N, K, per_row, cus);
@@ -3507,7 +3803,7 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
   // scales and more than 48 rows, the generic kernel.
   if (p.cfg == CFG_DECODE && !decode_offsets_ok(o.lda, o.ldb, M)) {
     if (per_row || M > 48) {
-      d.grid = ((N + 31) / 32) * ((M + 31) / 32);
+      resolve_generic(d, M, N, K, cus);
       return d;
     }
     p.cfg = CFG_SKINNY; p.bn = 16; p.splits = 1; p.kb_per_split = KB;
@@ -3554,7 +3850,7 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
       } else if (per_row) {
         d = Dispatch();
         d.per_row = true;
-        d.grid = ((N + 31) / 32) * ((M + 31) / 32);
+        resolve_generic(d, M, N, K, cus);
       } else {
         d.kernel = FP8B_KERNEL_BS128;
         d.waves = 8;
@@ -3577,7 +3873,7 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
       } else if (per_row) {
         d = Dispatch();
         d.per_row = true;
-        d.grid = ((N + 31) / 32) * ((M + 31) / 32);
+        resolve_generic(d, M, N, K, cus);
       } else {
         d.kernel = FP8B_KERNEL_BS128;
         d.waves = 4;
@@ -3951,12 +4247,14 @@ extern "C" int fp8b_w8a8_block_matmul(const void* A, int64_t lda, const void* B,
     g.lda = lda; g.ldb = ldb; g.as_sm = as_sm; g.as_sk = as_sk; g.bs_sn = bs_sn;
     g.bs_sk = bs_sk; g.ldc = ldc; g.M = M; g.N = N; g.K = K; g.block_n = block_n;
     g.block_k = block_k; g.out_dtype = out_dtype;
-    dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32));
+    g.KB = (K + block_k - 1) / block_k;
+    g.vec_store = ldc % 4 == 0 && ((uintptr_t)C & (esz == 4 ? 15 : 7)) == 0;
     if ((M + 31) / 32 > 65535) {
       set_error("fp8b_w8a8_block_matmul: M too large for the generic kernel");
       return FP8B_ERR_DIMS;
     }
-    gemm_generic_kernel<<<grid, 256, 0, st>>>(g);
+    if (block_n % 16 == 0) launch_generic<true>(g, d, st);
+    else launch_generic<false>(g, d, st);
     if (hipGetLastError() != hipSuccess) {
       set_error("fp8b_w8a8_block_matmul: generic kernel launch failed");
       return FP8B_ERR_LAUNCH;

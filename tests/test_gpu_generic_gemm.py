@@ -1,0 +1,89 @@
+"""The GEMM kernel for any block size, ragged K and unaligned rows (fp16 MFMAs on
+converted codes), at the sizes where its tiles, chunks and row ends can go
+wrong."""
+import pytest
+import torch
+
+from hf_kernels_helion_amd import deep_gemm_helion, finegrained_fp8_helion as fp8
+from hf_kernels_helion_amd.finegrained_fp8_helion import synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+def _offset_rows(t, pad, shift, dev):
+    """t as rows of a wider buffer, `shift` elements from its start."""
+    M, K = t.shape
+    buf = torch.zeros(M * (K + pad) + shift, dtype=torch.uint8, device=dev)
+    rows = buf.view(torch.float8_e4m3fn)[shift:].as_strided((M, K), (K + pad, 1))
+    rows.copy_(t.to(dev))
+    return rows
+
+
+def _exact(A, B, As, Bs, bn, bk):
+    """The formula in 64 bits, and the sum of its terms' magnitudes."""
+    K = A.shape[1]
+    a = A.double() * As.double().repeat_interleave(bk, 1)[:, :K]
+    b = B.double() * Bs.double().repeat_interleave(bn, 0)[:B.shape[0]].repeat_interleave(bk, 1)[:, :K]
+    return a @ b.t(), a.abs() @ b.abs().t()
+
+
+# Edges of the tile shapes (M 16 | 17, 32 | 33, few and many tiles), K one
+# byte around a 16-byte piece, a 128-byte chunk and a K-block, K below 16,
+# K-blocks of several chunks (block_k 256, 300), shorter than a piece
+# (block_k 8) and not a multiple of 16 (block_k 40), columns that share a
+# scale by 16 and not (block_n 128, 32, 24, 1), more waves than K-blocks.
+CASES = [(1, 1, 1, 128, 128), (3, 33, 15, 128, 128), (16, 40, 17, 128, 128),
+         (17, 65, 129, 128, 128), (16, 300, 1376, 128, 128), (33, 130, 255, 32, 128),
+         (40, 64, 300, 24, 64), (5, 70, 200, 1, 40), (20, 50, 90, 128, 8),
+         (64, 96, 1000, 1, 256), (31, 100, 700, 64, 300), (777, 4096, 1376, 128, 128),
+         (513, 8200, 143, 1, 128), (1030, 4100, 200, 48, 128), (9, 8225, 150, 128, 128),
+         (32, 4099, 385, 1, 128), (100, 3000, 333, 128, 128), (7, 100, 14, 16, 4)]
+
+
+@pytest.mark.parametrize("M,N,K,bn,bk", CASES)
+@pytest.mark.parametrize("pad,shift", [(0, 0), (3, 5), (16, 16)])
+def test_generic_gemm_keeps_fp32_sums(M, N, K, bn, bk, pad, shift, dev):
+    """fp32 output against 64 bits: every product is exact and every sum is in
+    fp32, so the error of a result is below (terms of a rounding chain) x
+    2^-24 of the sum of its terms' magnitudes: 8 roundings per 32 columns
+    inside a K-block, four per K-block for the fold. bf16 and fp16 outputs are
+    the fp32 ones rounded. Rows at any byte offset give the same bits."""
+    print(f"generic gemm {M}x{N}x{K} blocks {bn}x{bk} pad {pad} shift {shift}", flush=True)
+    A, B, As, Bs = synthetic.harness_operands(M, N, K, seed=M + N + K, block_n=bn, block_k=bk)
+    A, B = _offset_rows(A, pad, shift, dev), _offset_rows(B, pad, 2 * shift, dev)
+    As, Bs = As.to(dev), Bs.to(dev)
+    out = fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [bn, bk], torch.float32)
+    ref, mag = _exact(A, B, As, Bs, bn, bk)
+    chain = 8 * (min(bk, K) / 32 + 1) + 4 * (-(-K // bk))
+    if K % 128 or (bn, bk) not in ((128, 128), (1, 128)) or shift % 16 or pad % 16:
+        assert ((out.double() - ref).abs() <= chain * 2.0 ** -24 * mag).all()
+    for dtype in (torch.bfloat16, torch.float16):
+        assert torch.equal(fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [bn, bk], dtype),
+                           out.to(dtype))
+    if shift:
+        same = fp8.w8a8_block_fp8_matmul(A.contiguous(), B.contiguous(), As, Bs, [bn, bk],
+                                         torch.float32)
+        assert torch.equal(same, out)
+    if bn == 1:
+        assert torch.equal(deep_gemm_helion.gemm_fp8_fp8_bf16_nt(A, B, As, Bs, bk),
+                           out.to(torch.bfloat16))
+
+
+def test_generic_gemm_every_code_and_nan(dev):
+    """Each of the 256 codes against 1.0 comes back exactly (NaN as NaN), and
+    a NaN row, column or scale reaches only its own results."""
+    codes = torch.arange(256, dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn)
+    A = codes.view(256, 1).contiguous()
+    B = torch.ones(3, 1, device=dev).to(torch.float8_e4m3fn)
+    one = torch.ones(256, 1, device=dev)
+    out = fp8.w8a8_block_fp8_matmul(A, B, one, torch.ones(1, 1, device=dev), [128, 128],
+                                    torch.float32)
+    torch.testing.assert_close(out, codes.float().view(256, 1).expand(256, 3), rtol=0, atol=0,
+                               equal_nan=True)
+    A, B, As, Bs = [t.to(dev) for t in synthetic.harness_operands(40, 70, 143, seed=1)]
+    A.view(torch.uint8)[7, 142] = 0x7F
+    As[9, 1] = float("nan")
+    As[11, 0] = float("inf")
+    out = fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [128, 128], torch.float32)
+    bad = ~torch.isfinite(out)
+    assert bad[[7, 9, 11]].all() and not bad[[i for i in range(40) if i not in (7, 9, 11)]].any()
