@@ -76,6 +76,28 @@ py::object gemm_nt(py::handle A, py::handle B, py::handle As, py::handle Bs, int
   return py::cast(fp8b_torch::gemm_fp8_fp8_bf16_nt(T(A), T(B), T(As), T(Bs), block_k));
 }
 
+py::object weight_quant(py::handle W, int64_t block_n, int64_t block_k) {
+  if (!(plain_eager_tls() && plain_tensor(W))) return py::none();
+  return py::cast(fp8b_torch::weight_quant(T(W), block_n, block_k));
+}
+
+py::object gate_up_silu_quant(py::handle xq, py::handle xs, py::handle w, py::handle s,
+                              int64_t min_rows) {
+  if (!(plain_eager_tls() && plain_tensor(xq) && plain_tensor(xs) && plain_tensor(w) &&
+        plain_tensor(s)))
+    return py::none();
+  return py::cast(fp8b_torch::gate_up_silu_quant_rows(T(xq), T(xs), T(w), T(s), min_rows));
+}
+
+py::object fp8_mlp(py::handle x, py::handle wg, py::handle sg, py::handle wd, py::handle sd,
+                   int64_t bn, int64_t bk, bool fuse_quant, bool interleaved, int64_t min_rows) {
+  if (!(plain_eager_tls() && plain_tensor(x) && plain_tensor(wg) && plain_tensor(sg) &&
+        plain_tensor(wd) && plain_tensor(sd)))
+    return py::none();
+  return py::cast(fp8b_torch::fp8_mlp(T(x), T(wg), T(sg), T(wd), T(sd), bn, bk, fuse_quant,
+                                      interleaved, min_rows));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_fp8_fast, m) {
@@ -85,4 +107,7 @@ PYBIND11_MODULE(_fp8_fast, m) {
   m.def("silu_and_mul_quant", &silu_and_mul_quant);
   m.def("act_quant_matmul", &act_quant_matmul);
   m.def("gemm_fp8_fp8_bf16_nt", &gemm_nt);
+  m.def("weight_quant", &weight_quant);
+  m.def("gate_up_silu_quant", &gate_up_silu_quant);
+  m.def("fp8_mlp", &fp8_mlp);
 }

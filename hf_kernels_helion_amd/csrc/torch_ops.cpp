@@ -327,6 +327,73 @@ std::tuple<Tensor, Tensor> gate_up_silu_quant(const Tensor& A_in, const Tensor& 
   return {q, s};
 }
 
+// gate_up_silu_quant from min_rows rows, below that the GEMM and
+// silu_and_mul_quant on the interleaved layout (each 256-column block of the
+// GEMM's output is one gate | up pair).
+static void check_interleaved(int64_t k, const Tensor& w_il, bool two_d) {
+  TORCH_CHECK(two_d && w_il.dim() == 2 && w_il.size(0) % 256 == 0 && k % 128 == 0 && k != 0,
+              "gate_up_silu_quant: I must be a multiple of 128 and K a positive multiple of 128 "
+              "(K ", k, ", B ", w_il.sizes(), ")");
+}
+static std::tuple<Tensor, Tensor> silu_quant_interleaved(const Tensor& h) {
+  const int64_t m = h.size(0), i = h.size(1) / 2;
+  auto qs = silu_and_mul_quant(h.view({m * (i / 128), 256}), 128);
+  return {std::get<0>(qs).view({m, i}), std::get<1>(qs).view({m, i / 128})};
+}
+
+std::tuple<Tensor, Tensor> gate_up_silu_quant_rows(const Tensor& xq, const Tensor& xs,
+                                                   const Tensor& w_il, const Tensor& s_il,
+                                                   int64_t min_rows) {
+  TORCH_CHECK(xq.dim() >= 1, "xq must have at least one dimension");
+  const int64_t m = xq.size(0);
+  if (m >= min_rows || m == 0) return gate_up_silu_quant(xq, w_il, xs, s_il);
+  check_interleaved(xq.dim() == 2 ? xq.size(1) : 0, w_il, xq.dim() == 2);
+  return silu_quant_interleaved(matmul_impl(xq, w_il, xs, s_il, 128, 128, at::kBFloat16));
+}
+
+// The gated MLP of finegrained_fp8_helion/mlp.py in one host call: the same
+// launches and bits as its ops one by one, except that the gate/up GEMM
+// quantises bf16 activations itself (act_quant_matmul, the same bits again)
+// where its shapes allow, which saves a launch on decode-sized plans.
+Tensor fp8_mlp(const Tensor& x, const Tensor& w_gate_up, const Tensor& s_gate_up,
+               const Tensor& w_down, const Tensor& s_down, int64_t bn, int64_t bk,
+               bool fuse_quant, bool interleaved, int64_t min_rows) {
+  TORCH_CHECK(x.dim() >= 1, "x must have at least one dimension");
+  const int64_t k = x.size(-1);
+  const Tensor x2 = x.reshape({-1, k});
+  const int64_t m = x2.size(0);
+  Tensor hq, hs;
+  if (interleaved && (m >= min_rows || m == 0)) {
+    auto qs = act_quant(x2, bk);
+    std::tie(hq, hs) = gate_up_silu_quant(std::get<0>(qs), w_gate_up, std::get<1>(qs), s_gate_up);
+  } else {
+    const bool in_op = bn == 128 && bk == 128 && k % 128 == 0 && k > 0 && x2.is_cuda() &&
+                       x2.scalar_type() == at::kBFloat16;
+    Tensor h;
+    if (interleaved) check_interleaved(k, w_gate_up, true);
+    if (in_op) {
+      h = act_quant_matmul(x2, w_gate_up, s_gate_up, bn, bk, at::kBFloat16);
+    } else {
+      auto qs = act_quant(x2, bk);
+      h = matmul_impl(std::get<0>(qs), w_gate_up, std::get<1>(qs), s_gate_up, bn, bk,
+                      at::kBFloat16);
+    }
+    if (interleaved) {
+      std::tie(hq, hs) = silu_quant_interleaved(h);
+    } else if (fuse_quant) {
+      std::tie(hq, hs) = silu_and_mul_quant(h, bk);
+    } else {
+      Tensor a = at::empty({m, h.size(1) / 2}, h.options());
+      silu_and_mul(a, h);
+      std::tie(hq, hs) = act_quant(a, bk);
+    }
+  }
+  const Tensor y = matmul_impl(hq, w_down, hs, s_down, bn, bk, at::kBFloat16);
+  auto shape = x.sizes().vec();
+  shape.back() = y.size(1);
+  return y.view(shape);
+}
+
 // CPU tensors reach these: raise instead of computing anything.
 [[noreturn]] void no_cpu(const char* op) {
   TORCH_CHECK(false, op, ": tensors must be on a ROCm GPU; this package has no CPU "

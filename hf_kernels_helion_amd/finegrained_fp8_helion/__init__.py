@@ -106,6 +106,10 @@ def quantize_weight(W: torch.Tensor, block_size=(128, 128)):
     Bs = max(block amax, 1e-10) / 448 and Wq = e4m3fn(W / Bs) -- the (B, Bs)
     operands of w8a8_block_fp8_matmul and the weight/weight_scale_inv pair of
     FP8 checkpoints."""
+    if not _compiling():
+        r = _fast.weight_quant(W, int(block_size[0]), int(block_size[1]))
+        if r is not None:
+            return r
     return ops.weight_quant(W, int(block_size[0]), int(block_size[1]))
 
 

@@ -24,6 +24,7 @@ from __future__ import annotations
 import torch
 
 from ._ops import ops
+from .op import fast as _fast  # direct bindings for plain eager calls (None: take torch.ops)
 
 
 def interleave_gate_up(w_gate_up: torch.Tensor, s_gate_up: torch.Tensor):
@@ -54,6 +55,10 @@ def gate_up_silu_quant(xq: torch.Tensor, xs: torch.Tensor, w_il: torch.Tensor,
     runs unsplit), below that the chain's two ops on the interleaved layout.
     Needs block_size (128, 128) and H % 128 == 0. Returns (q [M, I] e4m3fn,
     s [M, I/128] fp32)."""
+    if not torch.compiler.is_compiling():
+        r = _fast.gate_up_silu_quant(xq, xs, w_il, s_il, FUSED_GATE_UP_MIN_ROWS)
+        if r is not None:
+            return r
     m = xq.shape[0]
     if m >= FUSED_GATE_UP_MIN_ROWS or m == 0:
         return ops.gate_up_silu_quant(xq, w_il, xs, s_il)
@@ -81,6 +86,14 @@ def fp8_mlp(x: torch.Tensor, w_gate_up: torch.Tensor, s_gate_up: torch.Tensor,
     default chain whenever its gate/up GEMM runs unsplit; below that many
     rows the default chain's ops on the interleaved layout, the same bits)."""
     bn, bk = int(block_size[0]), int(block_size[1])
+    # Plain eager calls run the chain in one C++ call, its gate/up GEMM
+    # quantising x itself (the same bits): the four ops below cost ~27 us of
+    # host time a call, more than a small MLP's kernels take.
+    if not torch.compiler.is_compiling() and (not gate_up_interleaved or (bn, bk) == (128, 128)):
+        y = _fast.fp8_mlp(x, w_gate_up, s_gate_up, w_down, s_down, bn, bk, bool(fuse_quant),
+                          bool(gate_up_interleaved), FUSED_GATE_UP_MIN_ROWS)
+        if y is not None:
+            return y
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1])
     xq, xs = ops.act_quant(x2, bk)
