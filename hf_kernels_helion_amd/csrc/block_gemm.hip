@@ -1453,6 +1453,47 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
   tile_epilogue<WM, WN>(a, smem, acc, m0 + wm * WM, n0 + wn * WN, wid, lane, split);
 }
 
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
+// 8 e4m3fn codes as fp16 (every code is exact, NaN stays NaN).
+__device__ __forceinline__ h8 fp8x8_to_f16(uint32_t lo, uint32_t hi) {
+  const h2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, false);
+  const h2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, true);
+  const h2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, false);
+  const h2 d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, true);
+  return h8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+// 16 bytes at any alignment (global loads need none on this target).
+__device__ __forceinline__ v4i load16_any(const uint8_t* p) {
+  v4i v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+// v without its first `skip` bytes, the following `valid` (0..16) bytes kept
+// and zeros after them.
+__device__ __forceinline__ v4i keep_bytes(const v4i v, int skip, int valid) {
+  uint64_t lo = (uint32_t)v[0] | ((uint64_t)(uint32_t)v[1] << 32);
+  uint64_t hi = (uint32_t)v[2] | ((uint64_t)(uint32_t)v[3] << 32);
+  if (skip >= 8) {
+    lo = hi >> (8 * (skip & 7));
+    hi = 0;
+  } else if (skip > 0) {
+    lo = (lo >> (8 * skip)) | (hi << (64 - 8 * skip));
+    hi >>= 8 * skip;
+  }
+  if (valid < 8) {
+    lo = valid <= 0 ? 0 : lo & ((uint64_t(1) << (8 * valid)) - 1);
+    hi = 0;
+  } else if (valid < 16) {
+    hi &= (uint64_t(1) << (8 * (valid - 8))) - 1;
+  }
+  return v4i{(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi,
+             (int)(uint32_t)(hi >> 32)};
+}
+
 // ---------------------------------------------------------------------------
 // Pipelined 128x128 kernel (grids below one 256x256 tile per CU, and the
 // split-K path). Waves of WM x WN (two per SIMD for 64x32); with half the operand
@@ -1473,7 +1514,17 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
 // scales read before the fragments (2%); level within 0.5%: DMA after odd
 // MFMAs, a raised wave priority over the first MFMAs.
 // ---------------------------------------------------------------------------
-template <int WM, int WN, bool PR>
+//
+// F16 (ragged K: a.KB counts the partial last K-block): the generic kernel's
+// fp32-exact sums at this kernel's pace. Fragments are converted to fp16 after
+// their LDS read, and a K-block is four 16x16x32 fp16 MFMAs per sub-tile,
+// summed in fp32 and folded once. The partial K-block's rows cannot come by
+// DMA (its 16-byte lanes would run past a row's end, and past the buffer's at
+// the last row): they go through registers, read at the row's last 16 bytes
+// where a piece crosses its end, bytes past K cleared. 1.2 us per K-block on
+// all CUs (750 TFLOP/s at 4096x4096x4080); a large bf16 product of the vendor's
+// library runs at 1347 on the same card, 0.8 us per K-block.
+template <int WM, int WN, bool PR, bool F16 = false>
 __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_kernel(GemmArgs a) {
   constexpr int BM = 128, BN = 128, NWN = BN / WN, NW = (BM / WM) * NWN;
   constexpr int FM = WM / 16, FN = WN / 16;
@@ -1575,10 +1626,38 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
         dma16_ptr(sbw_src + kk, lb + WIN_SA);
     }
   };
+  // F16: the partial last K-block through registers into stage `stage`. Its
+  // loads complete here, and so does every DMA issued before them.
+  const int kb_tail = F16 && (a.K & 127) != 0 ? a.KB - 1 : -1;
+  auto stage_tail = [&](int stage) {
+    v4i v[LPW];
+    int c16[LPW];
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) {
+      const int L = wid + i * NW;
+      const int Lr = i < A_LOADS ? L : L - BM / 8;
+      const int row = (Lr >> 3) * 64 + r8 * 8 + (Lr & 7);
+      c16[i] = kb_tail * 128 + ((lane & 7) ^ (Lr & 7)) * 16;
+      const uint8_t* p = i < A_LOADS ? a_base + (int64_t)min(row, a_lim) * a.lda
+                                     : b_base + (int64_t)min(row, b_lim) * a.ldb;
+      v[i] = load16_any(p + min(c16[i], a.K - 16));
+    }
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) {
+      const int valid = max(min(a.K - c16[i], 16), 0);
+      const int skip = valid > 0 ? c16[i] - min(c16[i], a.K - 16) : 0;  // 0..15
+      *reinterpret_cast<v4i*>(smem + stage * STAGE + (wid + i * NW) * 1024 + lane * 16) =
+          keep_bytes(v[i], skip, valid);
+    }
+  };
   // DMA of one K-block (and, at a window start, its scale window).
   auto issue_kb = [&](int kb) {
     const int rel = kb - kb_begin;
     if ((rel & 7) == 0) issue_win(kb, (rel >> 3) & 1);
+    if (F16 && kb == kb_tail) {
+      stage_tail(rel & (NSTAGE - 1));
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < LPW; ++i) issue_op(kb, rel & (NSTAGE - 1), i);
   };
@@ -1682,6 +1761,52 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
     // one instruction after every other MFMA
     const bool fill = KIND == 0 || (KIND == 1 && kb + NSTAGE < kb_end);
     const int rel_n = kb + NSTAGE - kb_begin;
+    if constexpr (F16) {
+      if (fill) issue_kb(kb + NSTAGE);
+      // Each step's converts run between the MFMAs of the step before (the
+      // waves of a SIMD move together, so the converts of one would otherwise
+      // meet the converts of the other), the next K-block's LDS reads between
+      // those of the first step, the folds two MFMAs behind in the last.
+      constexpr int NP = FM * FN;
+      static_assert(NP >= FM + FN + 1, "converts and reads fit between the MFMAs of a step");
+      v4f part[FM][FN];
+      h8 x[2][FM], w[2][FN];
+      auto convert = [&](int s, int f) {
+        const v8i& raw = f < FM ? xf[S][f] : wf[S][f - FM];
+        const h8 h = fp8x8_to_f16((uint32_t)raw[2 * s], (uint32_t)raw[2 * s + 1]);
+        if (f < FM) x[s & 1][f] = h;
+        else w[s & 1][f - FM] = h;
+      };
+      auto fold = [&](int q) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[q / FN][q % FN][e] =
+              fmaf(part[q / FN][q % FN][e], scale_of(S, q / FN, q % FN, e), acc[q / FN][q % FN][e]);
+      };
+#pragma unroll
+      for (int f = 0; f < FM + FN; ++f) convert(0, f);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          const int i = p / FN, j = p % FN;
+          part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              w[s & 1][j], x[s & 1][i], s == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : part[i][j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (s < 3 && p < FM + FN) convert(s + 1, p);
+          if constexpr (KIND < 2) {
+            if (s == 0 && p < FM + FN) read_frag(nst, T, p);
+            if (s == 1 && p == 0) read_scales(kb + 1, T);
+          }
+          if (s == 3 && p >= 2) fold(p - 2);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      fold(NP - 2);
+      fold(NP - 1);
+      if constexpr (KIND < 2) set_scales(T);
+      return;
+    }
     if (fill && (rel_n & 7) == 0) issue_win(kb + NSTAGE, (rel_n >> 3) & 1);
 #pragma unroll
     for (int p = 0; p < FM * FN; ++p) {
@@ -1742,7 +1867,7 @@ __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_ker
     body(kb, K0{}, K2{});
     last_set = 0;
   }
-  if (nkb > 0) {
+  if (!F16 && nkb > 0) {
     const int L = last_set;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -2895,47 +3020,6 @@ struct GenericArgs {
   int vec_store;  // four consecutive outputs can be stored as one vector
 };
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-
-// 8 e4m3fn codes as fp16 (every code is exact, NaN stays NaN).
-__device__ __forceinline__ h8 fp8x8_to_f16(uint32_t lo, uint32_t hi) {
-  const h2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, false);
-  const h2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, true);
-  const h2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, false);
-  const h2 d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, true);
-  return h8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
-}
-
-// 16 bytes at any alignment (global loads need none on this target).
-__device__ __forceinline__ v4i load16_any(const uint8_t* p) {
-  v4i v;
-  __builtin_memcpy(&v, p, 16);
-  return v;
-}
-
-// v without its first `skip` bytes, the following `valid` (0..16) bytes kept
-// and zeros after them.
-__device__ __forceinline__ v4i keep_bytes(const v4i v, int skip, int valid) {
-  uint64_t lo = (uint32_t)v[0] | ((uint64_t)(uint32_t)v[1] << 32);
-  uint64_t hi = (uint32_t)v[2] | ((uint64_t)(uint32_t)v[3] << 32);
-  if (skip >= 8) {
-    lo = hi >> (8 * (skip & 7));
-    hi = 0;
-  } else if (skip > 0) {
-    lo = (lo >> (8 * skip)) | (hi << (64 - 8 * skip));
-    hi >>= 8 * skip;
-  }
-  if (valid < 8) {
-    lo = valid <= 0 ? 0 : lo & ((uint64_t(1) << (8 * valid)) - 1);
-    hi = 0;
-  } else if (valid < 16) {
-    hi &= (uint64_t(1) << (8 * (valid - 8))) - 1;
-  }
-  return v4i{(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi,
-             (int)(uint32_t)(hi >> 32)};
-}
-
 // `n` (0..15) bytes at p one by one, zeros after them.
 __device__ __forceinline__ v4i load_bytes(const uint8_t* p, int n) {
   uint64_t lo = 0, hi = 0;
@@ -3110,7 +3194,7 @@ __global__ void __launch_bounds__(KW == 1 ? 256 : 64 * KW, 2) gemm_generic_kerne
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          acc[i][j][e] = fmaf(part[i][j][e] * sa[i], sb[j][BN16 ? 0 : e], acc[i][j][e]);
+          acc[i][j][e] = fmaf(part[i][j][e], sa[i] * sb[j][BN16 ? 0 : e], acc[i][j][e]);
   };
 
   if (kb_begin < kb_end) {
@@ -3627,9 +3711,9 @@ bool decode_offsets_ok(int64_t lda, int64_t ldb, int64_t M) {
 }
 
 bool mfma_path_ok(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M, int64_t N,
-                  int64_t K, int64_t block_n, int64_t block_k) {
-  return block_n == 128 && block_k == 128 && K % 128 == 0 && K > 0 && lda % 16 == 0 &&
-         ldb % 16 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0 &&
+                  int64_t K, int64_t block_n, int64_t block_k, bool ragged = false) {
+  return block_n == 128 && block_k == 128 && (ragged ? K % 128 != 0 && K >= 16 : K % 128 == 0) &&
+         K > 0 && lda % 16 == 0 && ldb % 16 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0 &&
          M < (int64_t(1) << 30) && N < (int64_t(1) << 30) && K < (int64_t(1) << 30);
 }
 
@@ -3637,6 +3721,7 @@ bool mfma_path_ok(const void* A, int64_t lda, const void* B, int64_t ldb, int64_
 struct Operands {
   int64_t lda, ldb;
   bool mfma;    // mfma_path_ok
+  bool ragged;  // all of it but whole K-blocks (K >= 16)
   bool scales;  // As, Bs contiguous in K with 16-byte aligned rows (16-byte window lanes)
 };
 
@@ -3649,6 +3734,7 @@ Operands contiguous_operands(int64_t M, int64_t N, int64_t K, int64_t block_n,
   const bool per_row = block_n == 1 && block_k == 128;
   o.mfma = K > 0 && K % 16 == 0 &&
            mfma_path_ok(nullptr, K, nullptr, K, M, N, K, per_row ? 128 : block_n, block_k);
+  o.ragged = mfma_path_ok(nullptr, K, nullptr, K, M, N, K, per_row ? 128 : block_n, block_k, true);
   o.scales = K % 512 == 0;  // K/128 scales per row: 16-byte rows when 4 | K/128
   return o;
 }
@@ -3778,6 +3864,17 @@ void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int cus) {
   else take(32, 32, tiles(32, 32) <= 2 * c ? 4 : 2);
 }
 
+// Ragged K on 16-byte aligned rows takes gemm_pipe128_kernel's fp16 form where
+// its tiles cover three quarters of the CUs: 777x4096x1376 (224 tiles) 19.3 us
+// against 22.8 on gemm_generic_kernel, 4096x4096x4080 181 against 211,
+// 300x8192x528 (192 tiles) 10.9 against 13.3; with half of the CUs
+// (400x4096x1376, 128 tiles) 18.4 against 16.5. Up to 64 rows most of a tile
+// is idle: 16x65536x528 21.5 against 16.2, 64x32768x1008 17.3 against 16.5
+// (100x28672x1008 16.7 against 18.7).
+bool ragged_pipe128(int64_t M, int64_t t128, int cus) {
+  return M > 64 && 4 * t128 >= 3 * (int64_t)cus;
+}
+
 template <bool BN16>
 void launch_generic(const GenericArgs& g, const Dispatch& d, hipStream_t st) {
   const dim3 grid((unsigned)((g.N + d.bn - 1) / d.bn), (unsigned)((g.M + d.bm - 1) / d.bm));
@@ -3796,7 +3893,17 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
   const bool per_row = block_n == 1 && block_k == 128;
   d.per_row = per_row;
   if (!o.mfma) {
-    resolve_generic(d, M, N, K, cus);
+    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
+    if (o.ragged && pipe_ok(o, K) && ragged_pipe128(M, t128, cus)) {
+      d.kernel = FP8B_KERNEL_PIPE128_F16;
+      d.bm = d.bn = 128;
+      d.waves = 8;
+      d.kb_per_split = (int)((K + 127) / 128);
+      d.grid = t128;
+      d.win4 = true;
+    } else {
+      resolve_generic(d, M, N, K, cus);
+    }
     return d;
   }
   const int KB = (int)(K / 128);
@@ -3897,21 +4004,22 @@ Dispatch resolve(int64_t M, int64_t N, int64_t K, int64_t block_n, int64_t block
   struct Entry {
     int64_t M = -1, N, K, bn, bk, lda, ldb;
     int cus;
-    bool mfma, scales;
+    bool mfma, ragged, scales;
     Dispatch d;
   };
   thread_local Entry cache[64];
   uint64_t h = (uint64_t)M * 0x9E3779B97F4A7C15ull ^ (uint64_t)N * 0xC2B2AE3D27D4EB4Full ^
                (uint64_t)K * 0x165667B19E3779F9ull ^ (uint64_t)block_n * 31 ^ (uint64_t)block_k ^
                (uint64_t)o.lda * 0x27D4EB2F165667C5ull ^ (uint64_t)o.ldb * 0x85EBCA77C2B2AE63ull ^
-               (uint64_t)cus << 7 ^ (uint64_t)o.mfma << 1 ^ (uint64_t)o.scales;
+               (uint64_t)cus << 7 ^ (uint64_t)o.mfma << 1 ^ (uint64_t)o.ragged << 2 ^ (uint64_t)o.scales;
   Entry& e = cache[(h ^ (h >> 29)) & 63];
   if (e.M == M && e.N == N && e.K == K && e.bn == block_n && e.bk == block_k && e.lda == o.lda &&
-      e.ldb == o.ldb && e.cus == cus && e.mfma == o.mfma && e.scales == o.scales)
+      e.ldb == o.ldb && e.cus == cus && e.mfma == o.mfma && e.ragged == o.ragged &&
+      e.scales == o.scales)
     return e.d;
   const Dispatch d = resolve_uncached(M, N, K, block_n, block_k, cus, o);
   e.M = M; e.N = N; e.K = K; e.bn = block_n; e.bk = block_k; e.lda = o.lda; e.ldb = o.ldb;
-  e.cus = cus; e.mfma = o.mfma; e.scales = o.scales; e.d = d;
+  e.cus = cus; e.mfma = o.mfma; e.ragged = o.ragged; e.scales = o.scales; e.d = d;
   return d;
 }
 
@@ -4071,6 +4179,9 @@ void launch_dispatch(const Dispatch& d, const GemmArgs& a, hipStream_t st) {
       if constexpr (PR) gemm_pipe128_kernel<64, 32, true><<<grid3, 512, 0, st>>>(a);
       else gemm_pipe128_kernel<32, 64, false><<<grid3, 512, 0, st>>>(a);
       break;
+    case FP8B_KERNEL_PIPE128_F16:
+      gemm_pipe128_kernel<32, 64, PR, true><<<grid3, 512, 0, st>>>(a);
+      break;
     case FP8B_KERNEL_BS128:
       if constexpr (!PR) {
         if (d.bm == 256) gemm_bs128_kernel<256, 256, 64, 128><<<grid3, 512, 0, st>>>(a);
@@ -4103,6 +4214,7 @@ const char* kernel_name(int k) {
     case FP8B_KERNEL_DECODE: return "gemm_decode_kernel";
     case FP8B_KERNEL_TINY: return "gemm_tiny_kernel";
     case FP8B_KERNEL_PIPE128: return "gemm_pipe128_kernel";
+    case FP8B_KERNEL_PIPE128_F16: return "gemm_pipe128_f16_kernel";
     case FP8B_KERNEL_PIPE256: return "gemm_pipe256_kernel";
     case FP8B_KERNEL_PIPE192: return "gemm_pipe192_kernel";
     case FP8B_KERNEL_PIPE256X128: return "gemm_pipe256x128_kernel";
@@ -4124,6 +4236,7 @@ Operands call_operands(const void* A, int64_t lda, const void* B, int64_t ldb, c
   o.lda = lda;
   o.ldb = ldb;
   o.mfma = mfma_path_ok(A, lda, B, ldb, M, N, K, per_row ? 128 : block_n, block_k);
+  o.ragged = mfma_path_ok(A, lda, B, ldb, M, N, K, per_row ? 128 : block_n, block_k, true);
   o.scales = as_sk == 1 && bs_sk == 1 && as_sm % 4 == 0 && bs_sn % 4 == 0 &&
              ((uintptr_t)As & 15) == 0 && ((uintptr_t)Bs & 15) == 0;
   return o;
@@ -4289,7 +4402,7 @@ extern "C" int fp8b_w8a8_block_matmul(const void* A, int64_t lda, const void* B,
   a.ws = (float*)workspace;
   a.lda = lda; a.ldb = ldb; a.as_sm = as_sm; a.as_sk = as_sk; a.bs_sn = bs_sn;
   a.bs_sk = bs_sk; a.ldc = ldc; a.M = (int)M; a.N = (int)N; a.K = (int)K;
-  a.KB = (int)(K / 128);
+  a.KB = (int)((K + 127) / 128);
   a.kb_per_split = d.kb_per_split;
   a.tiles_m = (int)tiles_m;
   a.tiles_n = (int)tiles_n;
@@ -4609,6 +4722,7 @@ extern "C" int fp8b_gate_up_silu_quant(const void* A, int64_t lda, const void* B
   o.lda = lda;
   o.ldb = ldb;
   o.mfma = true;
+  o.ragged = false;
   o.scales = as_sk == 1 && bs_sk == 1 && as_sm % 4 == 0 && bs_sn % 4 == 0 &&
              ((uintptr_t)As & 15) == 0 && ((uintptr_t)Bs & 15) == 0;
   a.win4 = win16_ok(o, K, 1, a.KB) ? 0 : 1;

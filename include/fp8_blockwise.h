@@ -106,8 +106,9 @@ int fp8b_act_quant_typed(const void* x, int64_t ldx, int x_dtype,
  * kb runs over ceil(K/block_k) K-blocks; nb over ceil(N/block_n).
  *
  * block_n = block_k = 128, K % 128 == 0, 16-byte aligned A/B with lda, ldb
- * multiples of 16 take the MFMA path; any other positive block sizes take a
- * generic (slower) GPU kernel with the same semantics.
+ * multiples of 16 take the fp8 MFMA path; any other positive block sizes, K
+ * and alignments take slower kernels with the same semantics (fp16 MFMAs on
+ * the converted codes, fp32 sums).
  * workspace may be NULL when fp8b_gemm_workspace_size() returns 0 for the
  * same arguments; otherwise it must hold at least that many bytes.
  */
@@ -128,7 +129,7 @@ size_t fp8b_gemm_workspace_size(int64_t M, int64_t N, int64_t K,
 /* Kernels of the GEMM plans (fp8b_plan_info.kernel, .tail_kernel). */
 typedef enum fp8b_kernel {
   FP8B_KERNEL_NONE = 0,
-  FP8B_KERNEL_GENERIC = 1,      /* SIMT fallback: any block size, unaligned operands */
+  FP8B_KERNEL_GENERIC = 1,      /* fp16 MFMAs: any block size, ragged K, unaligned operands */
   FP8B_KERNEL_SKINNY = 2,       /* M <= 48, 16 output columns x all of K per workgroup */
   FP8B_KERNEL_DECODE = 3,       /* M <= 64, 128 columns x a K split per workgroup */
   FP8B_KERNEL_TINY = 4,         /* small grids: 32x32, 32x16 or 64x64 tiles */
@@ -139,7 +140,8 @@ typedef enum fp8b_kernel {
   FP8B_KERNEL_BS128 = 9,        /* two-stage 128x128 / 256x256 tiles (FP8B_PIPE=0, huge leading dims) */
   FP8B_KERNEL_DECODE_QUANT = 10, /* fp8b_act_quant_matmul, M <= 32: act-quant inside the decode kernel */
   FP8B_KERNEL_SKINNY_QUANT = 11, /* fp8b_act_quant_matmul, M <= 8: act-quant inside the skinny kernel */
-  FP8B_KERNEL_TINY_QUANT = 12    /* fp8b_act_quant_matmul, M <= 8 (16 on short K): act-quant inside the small-grid kernel */
+  FP8B_KERNEL_TINY_QUANT = 12,   /* fp8b_act_quant_matmul, M <= 8 (16 on short K): act-quant inside the small-grid kernel */
+  FP8B_KERNEL_PIPE128_F16 = 13   /* ragged K on aligned rows: 128x128 tiles, fp16 MFMAs */
 } fp8b_kernel;
 
 /* What fp8b_w8a8_block_matmul launches for one call. */

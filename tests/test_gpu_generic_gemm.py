@@ -4,6 +4,7 @@ wrong."""
 import pytest
 import torch
 
+from hf_kernels_helion_amd import _native
 from hf_kernels_helion_amd import deep_gemm_helion, finegrained_fp8_helion as fp8
 from hf_kernels_helion_amd.finegrained_fp8_helion import synthetic
 
@@ -67,6 +68,45 @@ def test_generic_gemm_keeps_fp32_sums(M, N, K, bn, bk, pad, shift, dev):
     if bn == 1:
         assert torch.equal(deep_gemm_helion.gemm_fp8_fp8_bf16_nt(A, B, As, Bs, bk),
                            out.to(torch.bfloat16))
+
+
+# Aligned rows on a grid of at least 192 tiles of 128x128: the partial K-block
+# alone (K 16, 112), in the first four K-blocks (200, 496) and in the fifth,
+# sixth and twentieth (528, 640 + 16, 2544), K off a 16-byte piece on padded
+# rows (1001, 1337), edges of the last row and column tile, per-row scales.
+ALIGNED = [(1500, 2100, 16, 128, 0), (1500, 2100, 112, 128, 0), (777, 4096, 200, 128, 0),
+           (777, 4096, 496, 1, 0), (300, 8192, 528, 128, 0), (1300, 4000, 656, 1, 16),
+           (100, 28673, 144, 128, 0), (1000, 3100, 2544, 128, 32), (700, 5000, 1001, 128, 7),
+           (65, 25000, 1337, 1, 7), (1025, 3000, 17, 128, 15)]
+
+
+@pytest.mark.parametrize("M,N,K,bn,pad", ALIGNED)
+def test_ragged_k_on_128_tiles(M, N, K, bn, pad, dev):
+    """gemm_pipe128_kernel's fp16 form: the error bound above against 64 bits,
+    16-bit outputs the fp32 one rounded, the bits of the kernel that unaligned
+    rows of the same operands take, column-major scales included."""
+    print(f"ragged 128 tiles {M}x{N}x{K} bn={bn} pad {pad}", flush=True)
+    if pad == 0 and K % 16 == 0 and _native.gemm_plan(M, N, K, block_n=bn)["cu_count"] == 256:
+        assert _native.gemm_plan(M, N, K, block_n=bn)["kernel"] == "gemm_pipe128_f16_kernel"
+    A, B, As, Bs = synthetic.harness_operands(M, N, K, seed=M + N + K, block_n=bn)
+    A, B = _offset_rows(A, pad, 16, dev), _offset_rows(B, pad, 32, dev)
+    As, Bs = As.to(dev), Bs.to(dev)
+    out = fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [bn, 128], torch.float32)
+    ref, mag = _exact(A, B, As, Bs, bn, 128)
+    chain = 8 * (min(128, K) / 32 + 1) + 4 * (-(-K // 128))
+    assert ((out.double() - ref).abs() <= chain * 2.0 ** -24 * mag).all()
+    for dtype in (torch.bfloat16, torch.float16):
+        assert torch.equal(fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [bn, 128], dtype),
+                           out.to(dtype))
+    As_t, Bs_t = As.t().contiguous().t(), Bs.t().contiguous().t()
+    assert torch.equal(fp8.w8a8_block_fp8_matmul(A, B, As_t, Bs_t, [bn, 128], torch.float32), out)
+    off = fp8.w8a8_block_fp8_matmul(_offset_rows(A, 3, 1, dev), B, As, Bs, [bn, 128],
+                                    torch.float32)
+    if -(-M // 64) * -(-N // 128) >= 256:
+        assert torch.equal(off, out)  # both walk K in order
+    A.view(torch.uint8)[M - 1, K - 1] = 0x7F
+    bad = ~torch.isfinite(fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [bn, 128], torch.float32))
+    assert bad[M - 1].all() and not bad[:M - 1].any()
 
 
 def test_generic_gemm_every_code_and_nan(dev):
