@@ -1191,12 +1191,19 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
   constexpr int STAGE = (BM + BN) * 128;          // 48 KiB
   constexpr int LPW = (BM + BN) / 8 / NW;         // 6 wave-loads per wave per K-block
   constexpr int A_LOADS = BM / 64;                // wave-loads i < 4 bring A rows
+  // Three stages: two K-blocks of DMA in flight over the barrier instead of
+  // one: 4096x2048x4096 35.4 -> 33.9 us, 640x8192x8192 54.3 -> 52.2,
+  // 768x2000x14336 (split) 38.4 -> 35.1. They leave 16 KiB for the
+  // two windows of activation scales, so the weight scales, one per workgroup
+  // and K-block, sit in a register, 64 K-blocks one per lane; the per-row
+  // form's windows hold the weight rows too and leave room for two stages.
+  constexpr int NST = PR ? 2 : 3;
   constexpr int WIN_SA = BM * 32;
-  constexpr int WIN = WIN_SA + (PR ? 8 * BN * 4 : 256);
-  constexpr int SW_OFF = 2 * STAGE;
+  constexpr int WIN = WIN_SA + (PR ? 8 * BN * 4 : 0);
+  constexpr int SW_OFF = NST * STAGE;
   constexpr int EPI_PITCH = WN * 2 + 16;
   constexpr int EPI = NW * WM * EPI_PITCH;
-  constexpr int SMEM = (2 * STAGE + 2 * WIN > EPI) ? 2 * STAGE + 2 * WIN : EPI;
+  constexpr int SMEM = (SW_OFF + 2 * WIN > EPI) ? SW_OFF + 2 * WIN : EPI;
   constexpr int BAR = 8;                          // MFMA index of the barrier
   static_assert(SMEM <= 160 * 1024, "LDS budget");
   static_assert(LPW <= NP - BAR, "one DMA instruction per MFMA after the barrier");
@@ -1245,13 +1252,21 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
     }
   };
   // Scale window of 8 K-blocks: wave w brings As rows 32w..32w+31 (two lanes
-  // per row, 4 K-blocks each); lanes 0-1 of wave 7 also bring the tile's Bs
-  // row (PR: wave w brings slot w, the 128 rows' scales of K-block kb0 + w).
-  // With 16-byte lanes a half-window past kb_end re-reads the first half (KB
-  // is then a multiple of 4), so no lane reads past the row.
+  // per row, 4 K-blocks each; PR: and slot w, the 128 weight rows' scales of
+  // K-block kb0 + w). With 16-byte lanes a half-window past kb_end re-reads
+  // the first half (KB is then a multiple of 4), so no lane reads past the row.
   const float* saw_src =
       a.As + (int64_t)min(m0 + wid * 32 + (lane >> 1), a.M - 1) * a.as_sm + 4 * (lane & 1);
-  const float* sbw_src = a.Bs + (int64_t)(n0 >> 7) * a.bs_sn + 4 * (lane & 1);
+  // Weight scales of K-blocks kb..kb+63, one per lane. The empty asm makes the
+  // load complete here (with all DMA before it, once per 64 K-blocks), not at
+  // its later uses, where the wait would drain the DMA in flight each time.
+  float sb_lane = 0.f;
+  auto load_sb = [&](int kb) {
+    if constexpr (!PR) {
+      sb_lane = a.Bs[(int64_t)(n0 >> 7) * a.bs_sn + (int64_t)min(kb + lane, kb_end - 1) * a.bs_sk];
+      asm volatile("" : "+v"(sb_lane));
+    }
+  };
   auto issue_win = [&](int kb0, int wbuf) {
     const int kk = (kb0 + 4 * (lane & 1) < kb_end) ? kb0 : kb0 - 4 * (lane & 1);
     const uint32_t lb = lds0 + SW_OFF + wbuf * WIN;
@@ -1268,11 +1283,6 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
         dma4_ptr(a.Bs + (int64_t)min(row, a.N - 1) * a.bs_sn + (int64_t)kbs * a.bs_sk,
                  lb + WIN_SA + wid * 512 + h * 256);
       }
-    } else if (wid == NW - 1) {
-      if (a.win4)
-        win4_blocks(a.Bs, a.bs_sn, a.bs_sk, n0 >> 7, (a.N - 1) >> 7, 1, kb0, kb_end, lb + WIN_SA, lane);
-      else if (lane < 2)
-        dma16_ptr(sbw_src + kk, lb + WIN_SA);
     }
   };
 
@@ -1293,9 +1303,8 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
     return *reinterpret_cast<const float*>(smem + sa_off + o + i * 512);
   };
   auto rdsb = [&](int rel) {
-    if constexpr (PR) return 1.0f;
-    const int o = ((rel >> 3) & 1) * WIN + (rel & 7) * 4;
-    return *reinterpret_cast<const float*>(smem + SW_OFF + WIN_SA + o);
+    return PR ? 1.0f
+              : __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sb_lane), rel & 63));
   };
   // PR: the lane's four column scales of weight fragment j at K-block rel
   auto rdsbj = [&](int rel, int j) {
@@ -1313,47 +1322,55 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
   constexpr int ORD_I[NP] = {0, 1, 0, 1, 0, 1, 0, 1, 2, 3, 2, 3, 2, 3, 2, 3};
   constexpr int ORD_J[NP] = {0, 0, 1, 1, 2, 2, 3, 3, 0, 0, 1, 1, 2, 2, 3, 3};
   v8i w[FN], xs[FM];
-  float sc[FM], sa_t[FM], sb_n = 0.f;
+  float sc[FM], sa_t[FM];
   v4f sbj[PR ? FN : 1];
 #pragma unroll
   for (int j = 0; j < (PR ? FN : 1); ++j) sbj[j] = v4f{0.f, 0.f, 0.f, 0.f};
   v4f r1 = v4f{0.f, 0.f, 0.f, 0.f}, r2 = r1;  // results of MFMAs p-1 and p-2
 
   if (nkb > 0) {
+    load_sb(kb_begin);
 #pragma unroll
     for (int i = 0; i < LPW; ++i) issue_op(kb_begin, 0, i);
     issue_win(kb_begin, 0);
-    if (nkb > 1) {
 #pragma unroll
-      for (int i = 0; i < LPW; ++i) issue_op(kb_begin + 1, 1, i);
-      wait_vmcnt<LPW>();
-    } else {
-      wait_vmcnt<0>();
-    }
+    for (int u = 1; u < NST; ++u)
+      if (nkb > u) {
+#pragma unroll
+        for (int i = 0; i < LPW; ++i) issue_op(kb_begin + u, u, i);
+      }
+    if (nkb >= NST) wait_vmcnt<(NST - 1) * LPW>();
+    else if (nkb == 2) wait_vmcnt<LPW>();
+    else wait_vmcnt<0>();
     __syncthreads();
     w[0] = rdw(0, 0); w[1] = rdw(0, 1); w[2] = rdw(0, 2);
     xs[0] = rdx(0, 0); xs[1] = rdx(0, 1);
     sa_t[0] = rdsa(0, 0); sa_t[1] = rdsa(0, 1);
-    sb_n = rdsb(0);
     if constexpr (PR) { sbj[0] = rdsbj(0, 0); sbj[1] = rdsbj(0, 1); }
   }
 
-  // One K-block. KIND 0: steady state (reads the next K-block, DMA of
-  // kb+2); 1: next K-block exists but no kb+2; 2: last K-block. Empty asm
+  // One K-block, in stage st. KIND 0: steady state (reads the next K-block,
+  // DMA of kb+NST); 1: next K-block exists but no kb+NST; 2: last K-block. Empty asm
   // statements and sched_barrier keep the MFMAs, reads and folds in the
   // written order, as in gemm_pipe256_kernel.
+  int st = 0;
   auto body = [&](int kb, auto tag) {
     constexpr int KIND = decltype(tag)::value;
     const int rel = kb - kb_begin;
-    const int s = rel & 1;
-    const float sb = sb_n;
+    const int s = st, sn = st + 1 == NST ? 0 : st + 1;
+    st = sn;
+    if (!PR && rel > 0 && (rel & 63) == 0) load_sb(kb);
+    const float sb = rdsb(rel);
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       const int i = ORD_I[p], j = ORD_J[p];
       if (p == BAR && KIND < 2) {
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        // the DMA of kb+1 has landed; outstanding: kb+2's with three stages
+        if (KIND == 0 || (NST == 3 && kb + 2 < kb_end)) wait_vmcnt<(NST - 2) * LPW>();
+        else wait_vmcnt<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __syncthreads();
-        if (KIND == 0 && ((rel + 2) & 7) == 0) issue_win(kb + 2, ((rel + 2) >> 3) & 1);
+        if (KIND == 0 && ((rel + NST) & 7) == 0) issue_win(kb + NST, ((rel + NST) >> 3) & 1);
       }
       v4f res = mfma16x16x128(w[j], xs[i]);
       asm volatile("" : "+v"(res));
@@ -1372,14 +1389,14 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
       if (p == 1) { sc[0] = sa_t[0] * sb; sc[1] = sa_t[1] * sb; }
       if (p == 9) { sc[2] = sa_t[2] * sb; sc[3] = sa_t[3] * sb; }
       // after the barrier: the next K-block's rows 0-1 and weight fragments
-      // 0-2 (stage s^1) and the DMA of K-block kb+2 into stage s
+      // 0-2 (stage sn) and the DMA of K-block kb+NST into stage s
       if (KIND < 2 && p >= BAR) {
-        if (KIND == 0 && p - BAR < LPW) issue_op(kb + 2, s, p - BAR);
-        if (p == BAR) { xs[0] = rdx(s ^ 1, 0); sb_n = rdsb(rel + 1); sa_t[0] = rdsa(rel + 1, 0); }
-        if (p == BAR + 1) { xs[1] = rdx(s ^ 1, 1); sa_t[1] = rdsa(rel + 1, 1); }
-        if (p == BAR + 2) w[0] = rdw(s ^ 1, 0);
-        if (p == BAR + 4) w[1] = rdw(s ^ 1, 1);
-        if (p == BAR + 6) w[2] = rdw(s ^ 1, 2);
+        if (KIND == 0 && p - BAR < LPW) issue_op(kb + NST, s, p - BAR);
+        if (p == BAR) { xs[0] = rdx(sn, 0); sa_t[0] = rdsa(rel + 1, 0); }
+        if (p == BAR + 1) { xs[1] = rdx(sn, 1); sa_t[1] = rdsa(rel + 1, 1); }
+        if (p == BAR + 2) w[0] = rdw(sn, 0);
+        if (p == BAR + 4) w[1] = rdw(sn, 1);
+        if (p == BAR + 6) w[2] = rdw(sn, 2);
         // PR: the next K-block's column scales of fragments 0 and 1, after
         // this K-block's last folds with them (MFMAs 9 and 11)
         if constexpr (PR) {
@@ -1417,11 +1434,8 @@ __global__ void __launch_bounds__(512) gemm_pipe256x128_kernel(GemmArgs a) {
 #pragma unroll
   for (int i = 0; i < FM; ++i) sc[i] = 0.f;
   int kb = kb_begin;
-  for (; kb + 2 < kb_end; ++kb) body(kb, PipeKind<0>{});
-  if (kb + 1 < kb_end) {
-    body(kb, PipeKind<1>{});
-    ++kb;
-  }
+  for (; kb + NST < kb_end; ++kb) body(kb, PipeKind<0>{});
+  for (; kb + 1 < kb_end; ++kb) body(kb, PipeKind<1>{});
   if (kb < kb_end) {
     body(kb, PipeKind<2>{});
 #pragma unroll

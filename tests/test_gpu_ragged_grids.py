@@ -44,3 +44,30 @@ def test_every_tile_in_its_place(M, N, K, bn, dev):
     else:
         out = fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [128, 128], torch.float32)
         assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("KB", [1, 2, 3, 4, 5, 8, 9, 63, 64, 65, 66, 130])
+@pytest.mark.parametrize("strided", [False, True])
+def test_256x128_tiles_any_k_block_count(KB, strided, dev):
+    """gemm_pipe256x128_kernel's three stages over the shortest K ranges, the
+    ends of a scale window and of the 64 weight scales a register holds, with
+    scales in any layout: one-hot K-blocks against their exact scale products
+    (every K-block of A holds one 1.0, every one of B ones: the result is the
+    sum of As * Bs over the K-blocks, small powers of two, exact in fp32)."""
+    M, N, K = 2000, 3900, 128 * KB
+    p = _native.gemm_plan(M, N, K)
+    if p["cu_count"] == 256:
+        assert p["kernel"] == "gemm_pipe256x128_kernel", p
+    print(f"256x128 KB={KB} strided={strided}: {p['kernel']} splits {p['splits']}", flush=True)
+    A = torch.zeros(M, K, device=dev)
+    A[:, ::128] = 1.0
+    A = A.to(torch.float8_e4m3fn)
+    B = torch.ones(N, K, device=dev).to(torch.float8_e4m3fn)
+    g = torch.Generator().manual_seed(KB)
+    As = torch.exp2(torch.randint(0, 4, (M, KB), generator=g).float()).to(dev)
+    Bs = torch.exp2(torch.randint(0, 4, (-(-N // 128), KB), generator=g).float()).to(dev)
+    if strided:
+        As, Bs = As.t().contiguous().t(), Bs.t().contiguous().t()
+    out = fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [128, 128], torch.float32)
+    ref = (As.double() @ Bs.double().t()).repeat_interleave(128, 1)[:, :N].float()
+    assert torch.equal(out, ref)
