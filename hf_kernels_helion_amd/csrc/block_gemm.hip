@@ -1169,12 +1169,12 @@ __global__ void __launch_bounds__(512) gemm_pipe192_kernel(GemmArgs a) {
 //     barrier per K-block before MFMA 8 (every wave has read the whole
 //     current stage, and its DMA of the next stage has landed); after it the
 //     next K-block's rows 0-1 and weight fragments 0-2 are read into the
-//     registers their last use just freed, and the DMA of K-block kb+2 goes
-//     into the released stage, one instruction per MFMA.
+//     registers their last use just freed, and the DMA of K-block kb+3 (kb+2
+//     with PR) goes into the released stage, one instruction per MFMA.
 //   * Stage: 256 + 128 rows of 128 bytes (48 KiB) in the block layout of
-//     gemm_pipe256_kernel (A blocks 0-31, B blocks 32-47), two stages; scale
-//     windows of 8 K-blocks as there, with the tile's single weight-scale row
-//     (one scale per K-block for all 128 columns).
+//     gemm_pipe256_kernel (A blocks 0-31, B blocks 32-47), three stages (two
+//     with PR); activation scales in windows of 8 K-blocks as there, the
+//     tile's weight scales (one per K-block for all 128 columns) in a register.
 // PR (per-row weight scales, block_n = 1): as in gemm_pipe256_kernel, the
 // window holds the 128 weight rows' scales slot-major (4-byte DMA lanes) and
 // each fold multiplies the row scale by the lane's four column scales, read
@@ -3436,6 +3436,12 @@ bool use_fused_decode() {
 // within 2%).
 // FP8B_TILE192=0, FP8B_TILE256X128=0, FP8B_TAIL128=0 and FP8B_TAIL64=0
 // take the corresponding candidates out.
+// The fit predates the present K-block loops of the 128x128 (0.52-0.56 us per
+// K-block unsplit) and 256x128 kernels (0.91). Repricing 128x128 tiles at 0.56
+// (x1.10 per row, 64x64 quarters 0.47) moves 111 of 3276 swept shapes, mostly
+// long-K ones from split 256x128 to unsplit 128x128 tiles, to 0.90 of their
+// time (two slower, by 3 and 6%: 384 rows of per-row scales). The prices here
+// keep the long-K 256x128 split plans that callers and tests know.
 // ---------------------------------------------------------------------------
 struct TileCost {
   int cfg, bm, bn;
@@ -3884,9 +3890,10 @@ void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int cus) {
 // 300x8192x528 (192 tiles) 10.9 against 13.3; with half of the CUs
 // (400x4096x1376, 128 tiles) 18.4 against 16.5. Up to 64 rows most of a tile
 // is idle: 16x65536x528 21.5 against 16.2, 64x32768x1008 17.3 against 16.5
-// (100x28672x1008 16.7 against 18.7).
+// (100x28672x1008 16.7 against 18.7). Row counts that gemm_generic_kernel's
+// grid does not take are refused there.
 bool ragged_pipe128(int64_t M, int64_t t128, int cus) {
-  return M > 64 && 4 * t128 >= 3 * (int64_t)cus;
+  return M > 64 && (M + 31) / 32 <= 65535 && 4 * t128 >= 3 * (int64_t)cus;
 }
 
 template <bool BN16>
