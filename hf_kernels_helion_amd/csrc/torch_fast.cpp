@@ -7,8 +7,10 @@
 // returns None, so that the Python wrapper takes the torch.ops route, unless
 // the call is a plain eager one: every tensor argument exactly a
 // torch.Tensor (no subclass such as FakeTensor), none requiring grad, and no
-// TorchDispatchMode, torch-function mode or functorch transform active.
-// Results and errors are those of the torch.ops route (same functions).
+// TorchDispatchMode, torch-function mode, functorch transform or TorchScript
+// trace active (a trace would record the functions' at::empty and miss the
+// kernel that fills it). Results and errors are those of the torch.ops route
+// (same functions).
 #include <torch/extension.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -25,7 +27,8 @@ namespace {
 bool plain_eager_tls() {
   return c10::impl::TorchDispatchModeTLS::stack_len() == 0 &&
          !at::impl::torch_function_mode_enabled() &&
-         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
 
 bool plain_tensor(py::handle h) {

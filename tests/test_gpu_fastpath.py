@@ -100,6 +100,26 @@ def test_compiled_call_equals_eager(dev):
     torch._dynamo.reset()
 
 
+def test_traced_calls_equal_eager(dev):
+    """TorchScript traces of the public calls, run on inputs other than the
+    traced ones."""
+    A, B, As, Bs = _operands(64, 512, 512, dev)
+    W2, S2 = [t.to(dev) for t in synthetic.weights(512, 256, seed=5)]
+    fns = [lambda x: fp8.act_quant(x),
+           lambda x: fp8.act_quant_w8a8_block_fp8_matmul(x, B, Bs, [128, 128], torch.bfloat16),
+           lambda x: fp8.w8a8_block_fp8_matmul(*[A, B, fp8.act_quant(x)[1], Bs], [128, 128]),
+           lambda x: fp8.fp8_mlp(x, B, Bs, W2, S2),
+           lambda x: fp8.fp8_mlp(x, B, Bs, W2, S2, gate_up_interleaved=True),
+           lambda x: fp8.gate_up_silu_quant(*fp8.act_quant(x), B, Bs),
+           lambda x: fp8.quantize_weight(x)]
+    x0, x1 = [synthetic.activations(64, 512, seed=s).to(dev) for s in (1, 2)]
+    for i, f in enumerate(fns):
+        print(f"traced call {i}", flush=True)
+        a, b = torch.jit.trace(f, (x0,), check_trace=False)(x1), f(x1)
+        for u, v in zip(a, b) if isinstance(b, tuple) else [(a, b)]:
+            assert _same(u, v)
+
+
 def test_requires_grad_input_takes_the_op_route(dev):
     A, B, As, Bs = _operands(64, 256, 512, dev)
     As_g = As.clone().requires_grad_(True)

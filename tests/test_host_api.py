@@ -123,6 +123,44 @@ def test_public_api_compiles_to_the_registered_op():
     assert any("act_quant" in t for t in seen), seen
 
 
+def _binding_calls(dev="cpu"):
+    """One call of every direct binding, by name, and a tensor each of them takes."""
+    from hf_kernels_helion_amd.finegrained_fp8_helion import op
+    A, B = _fp8(7, 384, device=dev), _fp8(256, 384, device=dev)
+    As, Bs = torch.ones(7, 3, device=dev), torch.ones(2, 3, device=dev)
+    x = torch.zeros(7, 384, dtype=torch.bfloat16, device=dev)
+    down, sd = _fp8(384, 128, device=dev), torch.ones(3, 1, device=dev)
+    f = op.fast
+    return {
+        "w8a8_block_fp8_matmul_dtype": (lambda t: f.w8a8_block_fp8_matmul_dtype(
+            A, B, t, Bs, 128, 128, torch.bfloat16), As),
+        "act_quant": (lambda t: f.act_quant(t, 128), x),
+        "silu_and_mul": (lambda t: f.silu_and_mul(x[:, :192], t), x),
+        "silu_and_mul_quant": (lambda t: f.silu_and_mul_quant(t, 128), x),
+        "act_quant_matmul": (lambda t: f.act_quant_matmul(t, B, Bs, 128, 128, torch.bfloat16), x),
+        "gemm_fp8_fp8_bf16_nt": (lambda t: f.gemm_fp8_fp8_bf16_nt(
+            A, B, t, torch.ones(256, 3, device=dev), 128), As),
+        "weight_quant": (lambda t: f.weight_quant(t, 128, 128), x),
+        "gate_up_silu_quant": (lambda t: f.gate_up_silu_quant(A, t, B, Bs, 512), As),
+        "fp8_mlp": (lambda t: f.fp8_mlp(t, B, Bs, down, sd, 128, 128, True, False, 512), x),
+    }
+
+
+def test_direct_bindings_decline_while_tracing():
+    """A TorchScript trace records what the dispatcher sees: inside a binding
+    that is the output's allocation and not the kernel that fills it, so every
+    binding leaves a traced call to torch.ops."""
+    for name, (call, arg) in _binding_calls().items():
+        got = []
+
+        def f(t):
+            got.append(call(t))
+            return t + 1
+
+        torch.jit.trace(f, (arg,), check_trace=False)
+        assert got == [None], name
+
+
 def test_op_schemas_match_reference():
     # finegrained-fp8-helion/torch-ext/finegrained_fp8_helion/op.py:8-11 and
     # activation-helion/.../op.py:15-16
