@@ -5,8 +5,9 @@
 // boxes' hosts, more than a small GEMM or act-quant kernel runs. These
 // bindings call the same C++ op functions (torch_ops.h) without it. Each
 // returns None, so that the Python wrapper takes the torch.ops route, unless
-// the call is a plain eager one: every tensor argument exactly a
-// torch.Tensor (no subclass such as FakeTensor), none requiring grad, and no
+// the call is a plain eager one: every tensor argument exactly a dense
+// torch.Tensor (no subclass such as FakeTensor, no meta tensor, no negated
+// view), none requiring grad, and no
 // TorchDispatchMode, torch-function mode, functorch transform or TorchScript
 // trace active (a trace would record the functions' at::empty and miss the
 // kernel that fills it). Results and errors are those of the torch.ops route
@@ -31,8 +32,22 @@ bool plain_eager_tls() {
          !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
 
+// Whether the dispatcher would hand the op this tensor as it is: a dense CPU
+// or GPU tensor. Anything else is for the dispatcher to turn into one (a
+// negated or conjugated view, a zero tensor, a functional wrapper), to answer
+// (a meta tensor) or to refuse (sparse, nested).
+bool dense_tensor(const at::Tensor& t) {
+  using K = c10::DispatchKey;
+  constexpr c10::DispatchKeySet dense({K::CPU, K::CUDA, K::ADInplaceOrView, K::AutogradCPU,
+                                       K::AutogradCUDA, K::AutocastCPU, K::AutocastCUDA});
+  return (t.is_cuda() || t.is_cpu()) &&
+         ((t.key_set() - dense).raw_repr() & ~c10::full_backend_mask) == 0;
+}
+
 bool plain_tensor(py::handle h) {
-  return THPVariable_CheckExact(h.ptr()) && !THPVariable_Unpack(h.ptr()).requires_grad();
+  if (!THPVariable_CheckExact(h.ptr())) return false;
+  const at::Tensor& t = THPVariable_Unpack(h.ptr());
+  return !t.requires_grad() && dense_tensor(t);
 }
 
 const at::Tensor& T(py::handle h) { return THPVariable_Unpack(h.ptr()); }

@@ -120,6 +120,19 @@ def test_traced_calls_equal_eager(dev):
             assert _same(u, v)
 
 
+def test_negated_views_are_read_with_their_sign(dev):
+    x = torch.randn(16, 512, device=dev)
+    for v in (torch._neg_view(x), torch.complex(x, x).conj().imag, torch._neg_view(x[:, :1])):
+        assert v.is_neg()
+        for f in (fp8.act_quant, fp8.quantize_weight):
+            for a, b in zip(f(v), f(v.clone().resolve_neg())):
+                assert _same(a, b)
+    B, Bs = [t.to(dev) for t in synthetic.weights(512, 512, seed=5)]
+    W2, S2 = [t.to(dev) for t in synthetic.weights(512, 256, seed=6)]
+    xb = x.to(torch.bfloat16)
+    assert _same(fp8.fp8_mlp(torch._neg_view(xb), B, Bs, W2, S2), fp8.fp8_mlp(-xb, B, Bs, W2, S2))
+
+
 def test_requires_grad_input_takes_the_op_route(dev):
     A, B, As, Bs = _operands(64, 256, 512, dev)
     As_g = As.clone().requires_grad_(True)

@@ -161,6 +161,38 @@ def test_direct_bindings_decline_while_tracing():
         assert got == [None], name
 
 
+def test_direct_bindings_decline_tensors_the_dispatcher_rewrites():
+    """Meta tensors have the registered fake kernels' answer; a negated view or
+    an efficient zero tensor is one of its plain values only after the
+    dispatcher has made it so."""
+    for name, (call, arg) in _binding_calls().items():
+        for t in (torch.empty_like(arg, device="meta"), torch._neg_view(arg),
+                  torch._efficientzerotensor(arg.shape, dtype=arg.dtype),
+                  torch._to_functional_tensor(arg), arg.to_sparse()):
+            assert call(t) is None, (name, torch._C._dispatch_keys(t))
+        with pytest.raises(RuntimeError, match="ROCm GPU"):
+            call(torch.nn.Parameter(arg, requires_grad=False))
+
+
+def test_public_api_on_meta_tensors():
+    """Shapes and types without data or a GPU, as the registered ops give them."""
+    m = "meta"
+    W = torch.empty(300, 260, dtype=torch.bfloat16, device=m)
+    q, s = fp8.quantize_weight(W)
+    assert q.shape == W.shape and q.dtype == torch.float8_e4m3fn and s.shape == (3, 3)
+    x = torch.empty(2, 4, 256, dtype=torch.bfloat16, device=m)
+    wg, sg = _fp8(512, 256, device=m), torch.empty(4, 2, device=m)
+    wd, sd = _fp8(256, 256, device=m), torch.empty(2, 2, device=m)
+    for il in (False, True):
+        y = fp8.fp8_mlp(x, wg, sg, wd, sd, gate_up_interleaved=il)
+        assert y.shape == x.shape and y.dtype == torch.bfloat16 and y.is_meta
+    q, s = fp8.act_quant(x[0])
+    assert q.shape == (4, 256) and s.shape == (4, 2) and s.is_meta
+    q, s = fp8.gate_up_silu_quant(q, s, wg, sg)
+    assert q.shape == (4, 256) and s.shape == (4, 2)
+    assert fp8.w8a8_block_fp8_matmul(q, wd, s, sd, [128, 128]).shape == (4, 256)
+
+
 def test_op_schemas_match_reference():
     # finegrained-fp8-helion/torch-ext/finegrained_fp8_helion/op.py:8-11 and
     # activation-helion/.../op.py:15-16
