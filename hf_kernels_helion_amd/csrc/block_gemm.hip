@@ -3865,8 +3865,9 @@ void resolve_pipe128(Dispatch& d, int64_t tiles, int tail, int cus) {
 // per CU (64x4096x1376 6.1 against 7.5, 575x512x560 5.7 against 6.5). Up to 32
 // rows, 16x16 tiles with eight waves while they are at most two per CU
 // (16x4096x1376 4.1 against 5.7 us, 32x2048x1001 4.6 against 6.1), for more
-// columns 16x32 tiles up to 16 rows (8x8192x5000 10.8 against 12.1). K < 16
-// (rows read byte by byte): 32x32 tiles, four waves.
+// columns 16x32 tiles up to 16 rows (8x8192x5000 10.8 against 12.1) while their
+// 512 work-items each stay below the 2^32 that a launch takes along a grid
+// dimension (N < 2^28). K < 16 (rows read byte by byte): 32x32 tiles, four waves.
 void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int cus) {
   auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   auto take = [&](int bm, int bn, int waves) {
@@ -3879,7 +3880,7 @@ void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t c = cus;
   if (K < 16) take(32, 32, 4);
   else if (M <= 32 && tiles(16, 16) <= 2 * c) take(16, 16, 8);
-  else if (M <= 16) take(16, 32, 8);
+  else if (M <= 16 && tiles(16, 32) < (int64_t(1) << 23)) take(16, 32, 8);
   else if (tiles(64, 128) >= c) take(64, 128, 4);
   else take(32, 32, tiles(32, 32) <= 2 * c ? 4 : 2);
 }
@@ -3891,9 +3892,11 @@ void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int cus) {
 // (400x4096x1376, 128 tiles) 18.4 against 16.5. Up to 64 rows most of a tile
 // is idle: 16x65536x528 21.5 against 16.2, 64x32768x1008 17.3 against 16.5
 // (100x28672x1008 16.7 against 18.7). Row counts that gemm_generic_kernel's
-// grid does not take are refused there.
+// grid does not take are refused there, and 2^23 tiles or more, whose launch
+// would have 2^32 work-items in one dimension, run on its two-dimensional grid.
 bool ragged_pipe128(int64_t M, int64_t t128, int cus) {
-  return M > 64 && (M + 31) / 32 <= 65535 && 4 * t128 >= 3 * (int64_t)cus;
+  return M > 64 && (M + 31) / 32 <= 65535 && 4 * t128 >= 3 * (int64_t)cus &&
+         t128 < (int64_t(1) << 23);
 }
 
 template <bool BN16>

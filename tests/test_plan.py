@@ -90,6 +90,21 @@ def test_generic_plan_for_other_block_sizes():
     assert p["kernel"] == "gemm_generic_kernel" and p["splits"] == 1
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 65, 129, 257, 700])
+@pytest.mark.parametrize("N", [2 ** 28 - 40, 2 ** 28, 376_000_000, 2 ** 29 - 128, 2 ** 29 - 32])
+@pytest.mark.parametrize("K,block_n", [(9, 128), (17, 128), (48, 128), (48, 1), (1001, 64)])
+def test_wide_ragged_grids_stay_launchable(M, N, K, block_n):
+    """Launches of 2^32 work-items along a grid dimension or more are refused.
+    Block sizes and K that the fp8 MFMA kernels do not take run for every N up
+    to 32 * (2^24 - 1), whatever tile their rule picks."""
+    p = plan(M, N, K, block_n)
+    assert p["splits"] == 1 and p["tail_kernel"] == "none"
+    columns = -(-N // p["tile_n"])
+    grid_x = columns if p["kernel"] == "gemm_generic_kernel" else p["workgroups"]
+    assert p["workgroups"] == columns * -(-M // p["tile_m"])
+    assert grid_x * 64 * p["waves"] < 2 ** 32, p
+
+
 @pytest.mark.parametrize("M,I,K,kernel,tile_m", [
     (3001, 14336, 4096, "gemm_pipe192_kernel", 192),   # C5: 7 full waves of 192x256 tiles
     (1024, 8192, 512, "gemm_pipe256_kernel", 256),     # 256 tiles of 256x256: one wave
