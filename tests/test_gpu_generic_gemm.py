@@ -109,6 +109,32 @@ def test_ragged_k_on_128_tiles(M, N, K, bn, pad, dev):
     assert bad[M - 1].all() and not bad[:M - 1].any()
 
 
+# gemm_generic_kernel's tile rules and gemm_pipe128_kernel's fp16 form, with
+# scales shared by 16 columns and per column.
+@pytest.mark.parametrize("M,N,K,bn,bk", [(7, 40, 12, 128, 128), (16, 100, 200, 128, 128),
+                                         (9, 8225, 150, 1, 128), (200, 300, 333, 24, 64),
+                                         (777, 4096, 1001, 64, 128), (777, 4096, 208, 128, 128),
+                                         (777, 4096, 208, 1, 128)])
+@pytest.mark.parametrize("ea,eb,code", [(84, 45, 2.0 ** -8), (-100, -45, 256.0)])
+def test_scale_products_outside_fp32(M, N, K, bn, bk, ea, eb, code, dev):
+    """(sum * As) * Bs, the reference's order: each factor and the result are
+    normal fp32 numbers where As * Bs is infinite or subnormal, and a zero sum
+    stays zero. Against 64 bits, with the error bound above."""
+    print(f"extreme scales {M}x{N}x{K} blocks {bn}x{bk} 2^{ea} 2^{eb}", flush=True)
+    g = torch.Generator().manual_seed(M + K)
+    signs = lambda *s: torch.randint(0, 2, s, generator=g).float() * 2 - 1
+    A = (signs(M, K) * code).to(torch.float8_e4m3fn).to(dev)
+    B = (signs(N, K) * code).to(torch.float8_e4m3fn).to(dev)
+    A.view(torch.uint8)[M - 1] = 0
+    As = ((1 + torch.rand(M, -(-K // bk), generator=g)) * 2.0 ** ea).to(dev)
+    Bs = ((1 + torch.rand(-(-N // bn), -(-K // bk), generator=g)) * 2.0 ** eb).to(dev)
+    out = fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [bn, bk], torch.float32)
+    ref, mag = _exact(A, B, As, Bs, bn, bk)
+    chain = 8 * (min(bk, K) / 32 + 1) + 4 * (-(-K // bk))
+    assert ((out.double() - ref).abs() <= chain * 2.0 ** -24 * mag).all()
+    assert not out[M - 1].any()
+
+
 def test_generic_gemm_every_code_and_nan(dev):
     """Each of the 256 codes against 1.0 comes back exactly (NaN as NaN), and
     a NaN row, column or scale reaches only its own results."""
