@@ -3009,8 +3009,8 @@ splitk_reduce_xcd_kernel(GemmArgs a, int splits) {
 // range, 9.4e-9 against 1.0e-8 on normal ones).
 //
 // K is walked in chunks of 128 bytes that never cross a K-block, zero past
-// its end, and each chunk's sum is folded by itself (a K-block longer than 128
-// with the same scales for each of its chunks). A wave owns 16*FM activation rows x 16*FN weight rows. The rows of
+// its end; a K-block longer than 128 (LONG) keeps its sum over its chunks and
+// is folded once, at its last. A wave owns 16*FM activation rows x 16*FN weight rows. The rows of
 // a chunk go through registers into LDS (eight lanes of 16 bytes per row, at
 // any alignment; the next chunk and its scales are in flight while this one
 // is multiplied),
@@ -3056,8 +3056,8 @@ __device__ __forceinline__ v4i load_bytes(const uint8_t* p, int n) {
 
 // FM x FN fragments per wave. BN16: block_n is a multiple of 16, so a
 // fragment's columns share one weight scale (else one scale per column).
-// SHORT: K < 16, rows read byte by byte.
-template <int FM, int FN, int KW, bool BN16, bool SHORT = false>
+// SHORT: K < 16, rows read byte by byte. LONG: block_k > 128.
+template <int FM, int FN, int KW, bool BN16, bool SHORT = false, bool LONG = false>
 __global__ void __launch_bounds__(KW == 1 ? 256 : 64 * KW, 2) gemm_generic_kernel(GenericArgs g) {
   constexpr int NWM = KW == 1 ? 2 : 1, NWN = KW == 1 ? 2 : 1;
   constexpr int NSB = BN16 ? 1 : 4;      // weight scales per lane and fragment
@@ -3178,8 +3178,14 @@ __global__ void __launch_bounds__(KW == 1 ? 256 : 64 * KW, 2) gemm_generic_kerne
     return lds_frag2(p, ((2 * q) ^ sw) << 4, ((2 * q + 1) ^ sw) << 4);
   };
 
+  v4f part[FM][FN];  // sum of the K-block so far
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) part[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
   // One chunk from buffer buf.
   auto chunk = [&](int buf) {
+    const bool ends = !LONG || k_st + 128 >= kend_st;  // the last of its K-block
     float sa[FM], sb[FN][NSB];
 #pragma unroll
     for (int i = 0; i < FM; ++i) sa[i] = sa_n[i];
@@ -3193,7 +3199,6 @@ __global__ void __launch_bounds__(KW == 1 ? 256 : 64 * KW, 2) gemm_generic_kerne
     for (int i = 0; i < FM; ++i) xf[i] = frag(buf, (wm * FM + i) * 16);
 #pragma unroll
     for (int j = 0; j < FN; ++j) wf[j] = frag(buf, AR + (wn * FN + j) * 16);
-    v4f part[FM][FN];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       h8 x[FM], w[FN];
@@ -3208,15 +3213,18 @@ __global__ void __launch_bounds__(KW == 1 ? 256 : 64 * KW, 2) gemm_generic_kerne
 #pragma unroll
         for (int j = 0; j < FN; ++j)
           part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-              w[j], x[i], s == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : part[i][j], 0, 0, 0);
+              w[j], x[i], s == 0 && !LONG ? v4f{0.f, 0.f, 0.f, 0.f} : part[i][j], 0, 0, 0);
     }
+    if (!ends) return;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < FN; ++j) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           acc[i][j][e] = fmaf(part[i][j][e] * sa[i], sb[j][BN16 ? 0 : e], acc[i][j][e]);
+        if (LONG) part[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+      }
   };
 
   if (kb_begin < kb_end) {
@@ -3907,15 +3915,16 @@ bool ragged_pipe128(int64_t M, int64_t t128, int cus) {
          t128 < (int64_t(1) << 23);
 }
 
-template <bool BN16>
+template <bool BN16, bool LONG>
 void launch_generic(const GenericArgs& g, const Dispatch& d, hipStream_t st) {
   const dim3 grid((unsigned)((g.N + d.bn - 1) / d.bn), (unsigned)((g.M + d.bm - 1) / d.bm));
-  if (g.K < 16) gemm_generic_kernel<2, 2, 4, BN16, true><<<grid, 256, 0, st>>>(g);
-  else if (d.bn == 16) gemm_generic_kernel<1, 1, 8, BN16><<<grid, 512, 0, st>>>(g);
-  else if (d.bm == 16) gemm_generic_kernel<1, 2, 8, BN16><<<grid, 512, 0, st>>>(g);
-  else if (d.bm == 64) gemm_generic_kernel<2, 4, 1, BN16><<<grid, 256, 0, st>>>(g);
-  else if (d.waves == 4) gemm_generic_kernel<2, 2, 4, BN16><<<grid, 256, 0, st>>>(g);
-  else gemm_generic_kernel<2, 2, 2, BN16><<<grid, 128, 0, st>>>(g);
+  auto launch = [&](auto kernel) { kernel<<<grid, 64 * d.waves, 0, st>>>(g); };
+  if (g.K < 16) launch(gemm_generic_kernel<2, 2, 4, BN16, true>);
+  else if (d.bn == 16) launch(gemm_generic_kernel<1, 1, 8, BN16, false, LONG>);
+  else if (d.bm == 16) launch(gemm_generic_kernel<1, 2, 8, BN16, false, LONG>);
+  else if (d.bm == 64) launch(gemm_generic_kernel<2, 4, 1, BN16, false, LONG>);
+  else if (d.waves == 4) launch(gemm_generic_kernel<2, 2, 4, BN16, false, LONG>);
+  else launch(gemm_generic_kernel<2, 2, 2, BN16, false, LONG>);
 }
 
 // The launches of one GEMM call (see Dispatch) on a device with `cus` CUs.
@@ -4401,8 +4410,12 @@ extern "C" int fp8b_w8a8_block_matmul(const void* A, int64_t lda, const void* B,
       set_error("fp8b_w8a8_block_matmul: M too large for the generic kernel");
       return FP8B_ERR_DIMS;
     }
-    if (block_n % 16 == 0) launch_generic<true>(g, d, st);
-    else launch_generic<false>(g, d, st);
+    // (a single K-block is as long as K)
+    const bool bn16 = block_n % 16 == 0, lng = std::min(block_k, K) > 128;
+    if (bn16 && lng) launch_generic<true, true>(g, d, st);
+    else if (bn16) launch_generic<true, false>(g, d, st);
+    else if (lng) launch_generic<false, true>(g, d, st);
+    else launch_generic<false, false>(g, d, st);
     if (hipGetLastError() != hipSuccess) {
       set_error("fp8b_w8a8_block_matmul: generic kernel launch failed");
       return FP8B_ERR_LAUNCH;

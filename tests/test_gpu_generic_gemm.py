@@ -135,6 +135,31 @@ def test_scale_products_outside_fp32(M, N, K, bn, bk, ea, eb, code, dev):
     assert not out[M - 1].any()
 
 
+@pytest.mark.parametrize("M,N,K,bn,bk", [(5, 70, 600, 128, 256), (33, 130, 700, 1, 300),
+                                         (16, 8300, 384, 128, 257), (300, 6000, 512, 64, 512),
+                                         (700, 5000, 1000, 1, 256)])
+@pytest.mark.parametrize("exponent", [0, 112])
+def test_long_k_blocks_are_summed_before_scaling(M, N, K, bn, bk, exponent, dev):
+    """A K-block longer than 128 is one sum, scaled once: its halves cancel
+    exactly here but for the first column, with As * Bs so large at exponent 112
+    that either half scaled by itself is infinite."""
+    print(f"long K-blocks {M}x{N}x{K} blocks {bn}x{bk} 2^{exponent}", flush=True)
+    A = torch.full((M, K), 448.0)
+    k = torch.arange(K)
+    blk = k // bk * bk
+    size = torch.minimum(blk + bk, torch.tensor(K)) - blk
+    A[:, k - blk >= (size + 1) // 2] = -448.0
+    A[:, ((k - blk) == size // 2) & (size % 2 == 1)] = 0.0
+    A[:, 0] = 416.0
+    A = A.to(torch.float8_e4m3fn).to(dev)
+    B = torch.full((N, K), 448.0).to(torch.float8_e4m3fn).to(dev)
+    KB = -(-K // bk)
+    As = torch.full((M, KB), 2.0 ** (exponent // 2), device=dev)
+    Bs = torch.full((-(-N // bn), KB), 2.0 ** (exponent - exponent // 2), device=dev)
+    out = fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [bn, bk], torch.float32)
+    assert (out == -32.0 * 448.0 * 2.0 ** exponent).all()
+
+
 def test_generic_gemm_every_code_and_nan(dev):
     """Each of the 256 codes against 1.0 comes back exactly (NaN as NaN), and
     a NaN row, column or scale reaches only its own results."""
