@@ -3042,21 +3042,29 @@ struct GenericArgs {
   int vec_store;  // four consecutive outputs can be stored as one vector
 };
 
-// `n` (0..15) bytes at p one by one, zeros after them.
+// `n` (0..15) bytes at p, zeros after them: pieces of 8, 4, 2 and 1 bytes at
+// any alignment, whose loads do not wait for one another (one byte after the
+// other 176x768x13 took 17.3 us, 3.7 so).
 __device__ __forceinline__ v4i load_bytes(const uint8_t* p, int n) {
-  uint64_t lo = 0, hi = 0;
-#pragma unroll 1
-  for (int b = n - 1; b >= 0; --b) {
-    hi = (hi << 8) | (lo >> 56);
-    lo = (lo << 8) | p[b];
-  }
+  uint64_t head = 0, tail = 0;
+  uint32_t w4 = 0;
+  uint16_t w2 = 0;
+  uint8_t w1 = 0;
+  if (n & 8) __builtin_memcpy(&head, p, 8);
+  if (n & 4) __builtin_memcpy(&w4, p + (n & 8), 4);
+  if (n & 2) __builtin_memcpy(&w2, p + (n & 12), 2);
+  if (n & 1) w1 = p[n & 14];
+  if (n & 1) tail = w1;
+  if (n & 2) tail = tail << 16 | w2;
+  if (n & 4) tail = tail << 32 | w4;
+  const uint64_t lo = n & 8 ? head : tail, hi = n & 8 ? tail : 0;
   return v4i{(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi,
              (int)(uint32_t)(hi >> 32)};
 }
 
 // FM x FN fragments per wave. BN16: block_n is a multiple of 16, so a
 // fragment's columns share one weight scale (else one scale per column).
-// SHORT: K < 16, rows read byte by byte. LONG: block_k > 128.
+// SHORT: K < 16, rows read in pieces (load_bytes). LONG: block_k > 128.
 template <int FM, int FN, int KW, bool BN16, bool SHORT = false, bool LONG = false>
 __global__ void __launch_bounds__(KW == 1 ? 256 : 64 * KW, 2) gemm_generic_kernel(GenericArgs g) {
   constexpr int NWM = KW == 1 ? 2 : 1, NWN = KW == 1 ? 2 : 1;
@@ -3873,6 +3881,10 @@ void resolve_pipe128(Dispatch& d, int64_t tiles, int tail, int cus) {
   d.tail_grid = 4 * rest;
 }
 
+// Whether K is one chunk of gemm_generic_kernel (then there is nothing to split
+// over its waves).
+bool one_chunk(int64_t K, int64_t block_k) { return K <= std::min<int64_t>(block_k, 128); }
+
 // gemm_generic_kernel's tile (d.bm x d.bn) and waves. 64x128 tiles (2 x 2 waves
 // of 32x64) once they fill the CUs: 4096x4096x4080 213 us against 238 for
 // 64x64 tiles and 375 for 32x32 ones, 777x4096x1376 (416 tiles) 22.8 against
@@ -3883,8 +3895,11 @@ void resolve_pipe128(Dispatch& d, int64_t tiles, int tail, int cus) {
 // (16x4096x1376 4.1 against 5.7 us, 32x2048x1001 4.6 against 6.1), for more
 // columns 16x32 tiles up to 16 rows (8x8192x5000 10.8 against 12.1) while their
 // 512 work-items each stay below the 2^32 that a launch takes along a grid
-// dimension (N < 2^28). K < 16 (rows read byte by byte): 32x32 tiles, four waves.
-void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int cus) {
+// dimension (N < 2^28). K of one chunk or below 16 (rows read in pieces of 8, 4,
+// 2 and 1 bytes): no split along K, 32x32 tiles of 2 x 2 waves until 64x128 tiles
+// fill the CUs: with waves split along K all but one are idle there
+// (551x2171x20 10.1 us so, 6.2 unsplit; 4000x4000x12 123 and 25.5).
+void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int64_t block_k, int cus) {
   auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   auto take = [&](int bm, int bn, int waves) {
     d.kernel = FP8B_KERNEL_GENERIC;
@@ -3894,7 +3909,7 @@ void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int cus) {
     d.grid = tiles(bm, bn);
   };
   const int64_t c = cus;
-  if (K < 16) take(32, 32, 4);
+  if (K < 16 || one_chunk(K, block_k)) tiles(64, 128) >= c ? take(64, 128, 4) : take(32, 32, 4);
   else if (M <= 32 && tiles(16, 16) <= 2 * c) take(16, 16, 8);
   else if (M <= 16 && tiles(16, 32) < (int64_t(1) << 23)) take(16, 32, 8);
   else if (tiles(64, 128) >= c) take(64, 128, 4);
@@ -3919,7 +3934,9 @@ template <bool BN16, bool LONG>
 void launch_generic(const GenericArgs& g, const Dispatch& d, hipStream_t st) {
   const dim3 grid((unsigned)((g.N + d.bn - 1) / d.bn), (unsigned)((g.M + d.bm - 1) / d.bm));
   auto launch = [&](auto kernel) { kernel<<<grid, 64 * d.waves, 0, st>>>(g); };
-  if (g.K < 16) launch(gemm_generic_kernel<2, 2, 4, BN16, true>);
+  if (g.K < 16 && d.bm == 64) launch(gemm_generic_kernel<2, 4, 1, BN16, true>);
+  else if (g.K < 16) launch(gemm_generic_kernel<1, 1, 1, BN16, true>);
+  else if (one_chunk(g.K, g.block_k) && d.bm == 32) launch(gemm_generic_kernel<1, 1, 1, BN16>);
   else if (d.bn == 16) launch(gemm_generic_kernel<1, 1, 8, BN16, false, LONG>);
   else if (d.bm == 16) launch(gemm_generic_kernel<1, 2, 8, BN16, false, LONG>);
   else if (d.bm == 64) launch(gemm_generic_kernel<2, 4, 1, BN16, false, LONG>);
@@ -3943,7 +3960,7 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
       d.grid = t128;
       d.win4 = true;
     } else {
-      resolve_generic(d, M, N, K, cus);
+      resolve_generic(d, M, N, K, block_k, cus);
     }
     return d;
   }
@@ -3954,7 +3971,7 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
   // scales and more than 48 rows, the generic kernel.
   if (p.cfg == CFG_DECODE && !decode_offsets_ok(o.lda, o.ldb, M)) {
     if (per_row || M > 48) {
-      resolve_generic(d, M, N, K, cus);
+      resolve_generic(d, M, N, K, block_k, cus);
       return d;
     }
     p.cfg = CFG_SKINNY; p.bn = 16; p.splits = 1; p.kb_per_split = KB;
@@ -4001,7 +4018,7 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
       } else if (per_row) {
         d = Dispatch();
         d.per_row = true;
-        resolve_generic(d, M, N, K, cus);
+        resolve_generic(d, M, N, K, block_k, cus);
       } else {
         d.kernel = FP8B_KERNEL_BS128;
         d.waves = 8;
@@ -4024,7 +4041,7 @@ Dispatch resolve_uncached(int64_t M, int64_t N, int64_t K, int64_t block_n, int6
       } else if (per_row) {
         d = Dispatch();
         d.per_row = true;
-        resolve_generic(d, M, N, K, cus);
+        resolve_generic(d, M, N, K, block_k, cus);
       } else {
         d.kernel = FP8B_KERNEL_BS128;
         d.waves = 4;

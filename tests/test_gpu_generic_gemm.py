@@ -38,7 +38,10 @@ CASES = [(1, 1, 1, 128, 128), (3, 33, 15, 128, 128), (16, 40, 17, 128, 128),
          (40, 64, 300, 24, 64), (5, 70, 200, 1, 40), (20, 50, 90, 128, 8),
          (64, 96, 1000, 1, 256), (31, 100, 700, 64, 300), (777, 4096, 1376, 128, 128),
          (513, 8200, 143, 1, 128), (1030, 4100, 200, 48, 128), (9, 8225, 150, 128, 128),
-         (32, 4099, 385, 1, 128), (100, 3000, 333, 128, 128), (7, 100, 14, 16, 4)]
+         (32, 4099, 385, 1, 128), (100, 3000, 333, 128, 128), (7, 100, 14, 16, 4),
+         # one chunk and K < 16, on 32x32 tiles and (many tiles) 64x128 ones
+         (100, 130, 100, 1, 128), (33, 70, 128, 64, 128), (513, 8300, 13, 128, 128),
+         (1500, 3000, 11, 1, 4), (2000, 1300, 100, 24, 300), (700, 6000, 16, 1, 128)]
 
 
 @pytest.mark.parametrize("M,N,K,bn,bk", CASES)
