@@ -46,28 +46,37 @@ def test_every_tile_in_its_place(M, N, K, bn, dev):
         assert torch.equal(out, ref)
 
 
-@pytest.mark.parametrize("KB", [1, 2, 3, 4, 5, 8, 9, 63, 64, 65, 66, 130])
-@pytest.mark.parametrize("strided", [False, True])
-def test_256x128_tiles_any_k_block_count(KB, strided, dev):
-    """gemm_pipe256x128_kernel's three stages over the shortest K ranges, the
-    ends of a scale window and of the 64 weight scales a register holds, with
-    scales in any layout: one-hot K-blocks against their exact scale products
-    (every K-block of A holds one 1.0, every one of B ones: the result is the
-    sum of As * Bs over the K-blocks, small powers of two, exact in fp32)."""
-    M, N, K = 2000, 3900, 128 * KB
-    p = _native.gemm_plan(M, N, K)
-    if p["cu_count"] == 256:
-        assert p["kernel"] == "gemm_pipe256x128_kernel", p
-    print(f"256x128 KB={KB} strided={strided}: {p['kernel']} splits {p['splits']}", flush=True)
-    A = torch.zeros(M, K, device=dev)
-    A[:, ::128] = 1.0
-    A = A.to(torch.float8_e4m3fn)
-    B = torch.ones(N, K, device=dev).to(torch.float8_e4m3fn)
+# K-block counts: every number of stages in flight (up to 10), the ends of a
+# scale window (8) and of the 64 weight scales a register of the 256x128 kernel
+# holds, and odd and even totals of the 128x128 kernel's two register sets.
+K_BLOCKS = [*range(1, 11), 17, 63, 64, 65, 66, 130]
+
+
+@pytest.mark.parametrize("N,kernel", [(3900, "gemm_pipe256x128_kernel"),
+                                      (2000, "gemm_pipe128_kernel")])
+@pytest.mark.parametrize("bn", [128, 1])
+@pytest.mark.parametrize("KB", K_BLOCKS)
+def test_stages_any_k_block_count(KB, bn, N, kernel, dev):
+    """The pipelined 256x128 and 128x128 kernels over any number of K-blocks,
+    scales in either layout: random small integers, other ones in every row and
+    K-block, so that a fragment of another K-block, stage or row shows, and
+    power-of-two scales, other ones in every K-block. Every sum is a whole number
+    far below 2^24, which fp32 holds exactly in any order."""
+    M, K = 2000, 128 * KB
+    p = _native.gemm_plan(M, N, K, block_n=bn)
+    print(f"{M}x{N} KB={KB} bn={bn}: {p['kernel']} splits {p['splits']}", flush=True)
+    if p["cu_count"] == 256 and not (N == 2000 and KB == 130):  # (split 256x128 tiles)
+        assert (p["kernel"], p["splits"]) == (kernel, 1), p
     g = torch.Generator().manual_seed(KB)
+    ints = lambda rows: torch.randint(-4, 5, (rows, K), generator=g).float()
+    A, B = ints(M).to(dev), ints(N).to(dev)
     As = torch.exp2(torch.randint(0, 4, (M, KB), generator=g).float()).to(dev)
-    Bs = torch.exp2(torch.randint(0, 4, (-(-N // 128), KB), generator=g).float()).to(dev)
-    if strided:
-        As, Bs = As.t().contiguous().t(), Bs.t().contiguous().t()
-    out = fp8.w8a8_block_fp8_matmul(A, B, As, Bs, [128, 128], torch.float32)
-    ref = (As.double() @ Bs.double().t()).repeat_interleave(128, 1)[:, :N].float()
-    assert torch.equal(out, ref)
+    Bs = torch.exp2(torch.randint(0, 4, (-(-N // bn), KB), generator=g).float()).to(dev)
+    x = (A * As.repeat_interleave(128, 1)).double()
+    w = (B * Bs.repeat_interleave(bn, 0)[:N].repeat_interleave(128, 1)).double()
+    ref = x @ w.t()
+    assert ref.abs().max() < 2 ** 22
+    A8, B8 = A.to(torch.float8_e4m3fn), B.to(torch.float8_e4m3fn)
+    for As_l, Bs_l in ((As, Bs), (As.t().contiguous().t(), Bs.t().contiguous().t())):
+        out = fp8.w8a8_block_fp8_matmul(A8, B8, As_l, Bs_l, [bn, 128], torch.float32)
+        assert torch.equal(out.double(), ref)
