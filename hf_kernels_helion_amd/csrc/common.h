@@ -43,22 +43,6 @@ __device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
          ((uint32_t)__builtin_bit_cast(uint16_t, hb) << 16);
 }
 
-// Exact float8_e4m3fn -> fp32 decode (OCP E4M3: bias 7, no inf, S.1111.111 = NaN).
-__device__ __forceinline__ float fp8e4m3_to_f32(uint32_t b) {
-  const uint32_t sign = (b & 0x80u) << 24;
-  const uint32_t e = (b >> 3) & 0xFu;
-  const uint32_t m = b & 0x7u;
-  float v;
-  if (e == 0) {
-    v = (float)m * 0x1p-9f;
-  } else if (e == 15 && m == 7) {
-    v = __uint_as_float(0x7FC00000u);
-  } else {
-    v = __uint_as_float(((e + 120u) << 23) | (m << 20));
-  }
-  return __uint_as_float(__float_as_uint(v) | sign);
-}
-
 // Max over the 16 lanes of each DPP row (lanes 16r..16r+15) of an unsigned
 // value; every lane of the row receives the result.
 __device__ __forceinline__ uint32_t row16_max_u32(uint32_t v) {
