@@ -1521,13 +1521,13 @@ __device__ __forceinline__ v4i keep_bytes(const v4i v, int skip, int valid) {
 // the LDS reads alone 0.23, the DMA alone 0.36 (timing-only builds at
 // 1000x4096x7168), and together 0.52: LDS reads and DMA writes share the LDS
 // while two waves per SIMD share the matrix core. 0.63 before the K-block
-// body was free of branches (2048x2048x4096 25.1 -> 20.9 us, 1000x4096x7168
-// with fp32 output 42.0 -> 35.2). Measured slower: four waves of 64x64 (two
+// body was free of branches (calls on three operand sets in turn:
+// 2048x2048x4096 24.9 -> 21.6 us, 1000x4096x7168 with fp32 output 41.8 -> 35.1;
+// the kernel alone, few calls after idle, traces at 22.1 and 36.2). Measured slower: four waves of 64x64 (two
 // thirds of the LDS reads, but one wave per SIMD: 28.5 against 23.2 us at
 // 2048x2048x4096), all DMA of a K-block right after its barrier (2%), the
 // scales read before the fragments (2%); level within 0.5%: DMA after odd
 // MFMAs, a raised wave priority over the first MFMAs.
-// ---------------------------------------------------------------------------
 //
 // F16 (ragged K: a.KB counts the partial last K-block): the generic kernel's
 // fp32-exact sums at this kernel's pace. Fragments are converted to fp16 after
@@ -1535,9 +1535,13 @@ __device__ __forceinline__ v4i keep_bytes(const v4i v, int skip, int valid) {
 // summed in fp32 and folded once. The partial K-block's rows cannot come by
 // DMA (its 16-byte lanes would run past a row's end, and past the buffer's at
 // the last row): they go through registers, read at the row's last 16 bytes
-// where a piece crosses its end, bytes past K cleared. 1.2 us per K-block on
-// all CUs (750 TFLOP/s at 4096x4096x4080); a large bf16 product of the vendor's
-// library runs at 1347 on the same card, 0.8 us per K-block.
+// where a piece crosses its end, bytes past K cleared. Bound by the converts
+// and folds beside the MFMAs: 1.35 us for each further K-block of the 1024
+// tiles of 4096x4096 (four per CU; slope from K = 2032 to 8176), 189 us or 726
+// TFLOP/s in all at K = 4080, 1.47 us per K-block; the vendor's bf16 product
+// of 4096x4096x4096 takes 99 us on the same card, 0.77 us per 128x128x128, 0.71
+// by the slope.
+// ---------------------------------------------------------------------------
 template <int WM, int WN, bool PR, bool F16 = false>
 __global__ void __launch_bounds__((128 / WM) * (128 / WN) * 64) gemm_pipe128_kernel(GemmArgs a) {
   constexpr int BM = 128, BN = 128, NWN = BN / WN, NW = (BM / WM) * NWN;
@@ -3010,24 +3014,24 @@ splitk_reduce_xcd_kernel(GemmArgs a, int splits) {
 //
 // K is walked in chunks of 128 bytes that never cross a K-block, zero past
 // its end; a K-block longer than 128 (LONG) keeps its sum over its chunks and
-// is folded once, at its last. A wave owns 16*FM activation rows x 16*FN weight rows. The rows of
-// a chunk go through registers into LDS (eight lanes of 16 bytes per row, at
-// any alignment; the next chunk and its scales are in flight while this one
-// is multiplied),
-// 16-byte piece c of row R in slot c ^ (R/2 % 8), so that the fragment reads
-// (16 rows, one piece) meet distinct banks; fragments are converted after the
-// read. Lane l holds bytes 32*(l/16)..+31 of row l%16 of a fragment, and step
+// is folded once, at its last. A wave owns 16*FM activation rows x 16*FN
+// weight rows. The rows of a chunk go through registers into LDS (eight lanes
+// of 16 bytes per row, at any alignment; the next chunk and its scales are in
+// flight while this one is multiplied), 16-byte piece c of row R in slot
+// c ^ (R/2 % 8), so that the fragment reads (16 rows, one piece) meet distinct
+// banks; fragments are converted after the read. Lane l holds bytes 32*(l/16)..+31 of row l%16 of a fragment, and step
 // s of a chunk multiplies bytes 8s..8s+7 of every lane, the same K for both
 // operands. KW = 1: four waves on 2 x 2 tiles share two LDS buffers, one
 // barrier per chunk. KW > 1 (few rows or few tiles): each wave stages its own
 // rows, without barriers, the waves split the K-blocks of one tile and sum
 // through LDS in wave order.
 // Bound: converts, folds and MFMAs of two waves per SIMD, which overlap only
-// in part (0.85 us per 64x128 tile and chunk and CU, 0.21 of it MFMAs):
-// 4096x4096x4080 213 us (645 TFLOP/s), 777x4096x1376 22.8 us against 330 on
-// the SIMT kernel this replaces. Measured slower: fragments straight from
-// global memory without LDS (43.5 us at 777x4096x1376: four cache lines per
-// four lanes), loads two chunks ahead (25.5 us), 128x128 tiles (46.7).
+// in part (0.87 us per 64x128 tile and chunk and CU, 0.21 of it MFMAs):
+// 4096x4096x4080 223 us (614 TFLOP/s) on aligned rows, 270 on rows one byte off,
+// 777x4096x1376 23.8 and 29.1 us against 330 on the SIMT kernel this replaces.
+// Measured slower at 777x4096x1376: fragments straight from global memory
+// without LDS (43.5 us: four cache lines per four lanes), loads two chunks
+// ahead (25.5), 128x128 tiles (46.7).
 // ---------------------------------------------------------------------------
 struct GenericArgs {
   const uint8_t* A;
@@ -3422,50 +3426,50 @@ bool use_fused_decode() {
 //   + K-blocks x time per K-block of the tile x the wave's power factor
 //   + the wave's output stores,
 // plus, for a K split, the fp32 partials and the split-K sum kernel; the
-// cheapest wins. Time per K-block of one tile on one CU of a fully busy
-// chip (MI355X, realistic operand bits, power-limited clock): 256x256
-// 1.72 us, 192x256 1.37, 256x128 0.95, 128x128 0.71; 64x64 quarters on the
-// small-grid kernel 0.40. A wave that keeps a fraction f of the CUs busy
-// runs each tile faster, the power limit then allowing a higher clock:
-// factor max(0.8, 1 - 0.8 (1 - f)) (a 192-tile wave of 256x256 tiles takes
-// 1.41 us per K-block). The model reproduces the measured order of the
-// plans it chooses between, e.g. (us, steady clock):
-//   3001x4096x14336   192x256 one wave 157.8 < 256x256 partial wave 160.3
-//                     < 128x128 three waves 241
-//   3001x28672x4096   256x256 + last wave as 128x128 quarters 320.3
-//                     < 192x256 seven waves 331.4
-//   2048x4096x4096    256x128 one wave 34.8 < 128x128 two waves 47.1
-//   2048x2048x4096    128x128 one wave 25.3 < 256x128 half a wave 30.1
-//   2048x6144x4096    256x256 partial wave 47.1 < 256x128 two waves 61.2
-//   4096x6144x14336   256x256 + last wave as 256x128 halves 298.9
-//                     < 256x256 two waves 326.0
-//   2048x2560x4096    128x128 + last wave as 64x64 quarters 37.9
-//                     < 128x128 two waves 45.3
-//   1024x4096x14336   256x128 split in two 69.6 < 128x128 one wave 75.2
-//   512x4096x14336    256x128 split four ways 44.4 < 128x128 split two 51.7
+// cheapest wins. kTileCosts holds the time per K-block of one tile on one CU of
+// a fully busy chip (MI355X, realistic operand bits, power-limited clock). A
+// wave that keeps only some of the CUs busy runs each tile faster, the power
+// limit then allowing a higher clock (power_factor). The order of the plans it
+// chooses between, measured (us, operands streamed from HBM):
+//   3001x4096x14336   192x256 one wave 163.6 < 256x256 partial wave 176.5
+//                     < 128x128 three waves 203.7
+//   3001x28672x4096   256x256 + last wave as 128x128 quarters 323.2
+//                     < 192x256 seven waves 346.2
+//   2048x4096x4096    256x128 one wave 39.7 < 128x128 two waves 46.7
+//   2048x2048x4096    128x128 one wave 24.5 < 256x128 half a wave 34.8
+//   2048x6144x4096    256x256 partial wave 56.3 < 256x128 two waves 65.9
+//                     < 128x128 three waves 68.1
+//   4096x6144x14336   256x256 + last wave as 256x128 halves 315.0
+//                     < 256x256 two waves 342.7
+//   2048x2560x4096    256x128 partial wave 34.4 < 128x128 + last wave as
+//                     64x64 quarters 38.1 < 128x128 two waves 43.3
+//   1024x4096x14336   128x128 one wave 74.8 < 256x128 split in two 76.1
+//   512x4096x14336    256x128 split four ways 47.4 < 128x128 split two 48.1
 // A K split is considered only while the split grid fits one wave of
-// workgroups (a second wave costs more than the idle CUs: 1536x1536x4096
-// 40.2 us split in two, 24.2 unsplit); 256x256 and 192x256 grids are never
-// split. Two exclusions the model does not reproduce, each measured on
-// several shapes with the weights streamed from HBM: 256x128 tiles are not
-// split over 8 or fewer column tiles (N = 1024: 2048x1024x14336 56.0 us
-// split four ways against 48.1 for 128x128 tiles split two ways,
-// 1536x1024x14336 49.5 against 45.8, 1280x1024x14336 47.6 against 44.7),
-// nor below 256 rows (M = 200: 200x14336x14336 82.0 split two ways against
-// 76.6 on 128x128 tiles, 200x16384x14336 86.0 against 81.6, 200x11008x14336
-// 77.5 against 74.5; unsplit they stay ahead: 200x28672x4096 47.0 against
-// 53.0 on 192x256 tiles). Per-row weight scales (one more multiply per
-// fold) slow the tiles unevenly: x1.10 for 256x256, x1.08 for 256x128,
-// x1.20 for 128x128 (fitted to 72 shapes, 69 of their 72 choices right or
-// within 2%).
+// workgroups (a second wave costs more than the idle CUs); 256x256 and 192x256
+// grids are never split. Two exclusions the model does not reproduce: 256x128
+// tiles are not split over 8 or fewer column tiles (N = 1024:
+// 2048x1024x14336 54.7 us split four ways against 48.6 for 128x128 tiles
+// split two ways, 1536x1024x14336 44.8 both, but 1280x1024x14336 42.3 against
+// 44.0), nor below 256 rows. The second was drawn for a slower 256x128 loop
+// (200x14336x14336 82.0 split two ways against 76.6 on 128x128 tiles); with
+// the present one the split is ahead there (74.1 against 76.4, 200x16384x14336
+// 80.7 against 82.1, 200x11008x14336 64.2 against 69.4). Unsplit, 256x128
+// tiles stay ahead below 256 rows: 200x28672x4096 40.1 against 52.8 on 192x256
+// tiles. Per-row weight scales (one more multiply per fold) slow the tiles
+// unevenly: x1.10 for 256x256, x1.08 for 256x128, x1.20 for 128x128.
 // FP8B_TILE192=0, FP8B_TILE256X128=0, FP8B_TAIL128=0 and FP8B_TAIL64=0
 // take the corresponding candidates out.
-// The fit predates the present K-block loops of the 128x128 (0.52-0.56 us per
-// K-block unsplit) and 256x128 kernels (0.91). Repricing 128x128 tiles at 0.56
-// (x1.10 per row, 64x64 quarters 0.47) moves 111 of 3276 swept shapes, mostly
-// long-K ones from split 256x128 to unsplit 128x128 tiles, to 0.90 of their
-// time (two slower, by 3 and 6%: 384 rows of per-row scales). The prices here
-// keep the long-K 256x128 split plans that callers and tests know.
+// The prices were fitted together (247 timed plans, 4% RMS) to earlier K-block
+// loops of the 128x128 and 256x128 kernels, which have since become faster:
+// slopes over K (2048x2048 and 2048x4096, 32 to 64 K-blocks) give 0.56 us for
+// 128x128 tiles (priced 0.67), 0.92 for 256x128 (1.08), and per row 0.64 and
+// 1.28 (0.80, 1.17). The two prices fell by the same share, so the order
+// between these tiles mostly holds; against the 256x256 and 192x256 tiles,
+// the 64x64 quarters and between split and unsplit plans it is off by up to
+// that share (and the second exclusion above has lost its reason). Only a
+// refit of all prices at once would mend that: changing one tile's price
+// alone measures that tile against the others' old ones.
 // ---------------------------------------------------------------------------
 struct TileCost {
   int cfg, bm, bn;
@@ -3757,8 +3761,9 @@ bool decode_offsets_ok(int64_t lda, int64_t ldb, int64_t M) {
 bool mfma_path_ok(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M, int64_t N,
                   int64_t K, int64_t block_n, int64_t block_k, bool ragged = false) {
   return block_n == 128 && block_k == 128 && (ragged ? K % 128 != 0 && K >= 16 : K % 128 == 0) &&
-         K > 0 && lda % 16 == 0 && ldb % 16 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0 &&
-         M < (int64_t(1) << 30) && N < (int64_t(1) << 30) && K < (int64_t(1) << 30);
+         K > 0 && lda % 16 == 0 && ldb % 16 == 0 && ((uintptr_t)A & 15) == 0 &&
+         ((uintptr_t)B & 15) == 0 && M < (int64_t(1) << 30) &&
+         N < (int64_t(1) << 30) && K < (int64_t(1) << 30);
 }
 
 // Operand properties the kernel choice depends on, besides the sizes.
@@ -3885,19 +3890,21 @@ void resolve_pipe128(Dispatch& d, int64_t tiles, int tail, int cus) {
 // over its waves).
 bool one_chunk(int64_t K, int64_t block_k) { return K <= std::min<int64_t>(block_k, 128); }
 
-// gemm_generic_kernel's tile (d.bm x d.bn) and waves. 64x128 tiles (2 x 2 waves
-// of 32x64) once they fill the CUs: 4096x4096x4080 213 us against 238 for
-// 64x64 tiles and 375 for 32x32 ones, 777x4096x1376 (416 tiles) 22.8 against
-// 22.8 and 27.7. Below that 32x32 tiles with two waves along K (200x4096x1376
-// 10.1 us against 12.4 on 64x64 tiles), four where the tiles are at most two
-// per CU (64x4096x1376 6.1 against 7.5, 575x512x560 5.7 against 6.5). Up to 32
-// rows, 16x16 tiles with eight waves while they are at most two per CU
-// (16x4096x1376 4.1 against 5.7 us, 32x2048x1001 4.6 against 6.1), for more
-// columns 16x32 tiles up to 16 rows (8x8192x5000 10.8 against 12.1) while their
-// 512 work-items each stay below the 2^32 that a launch takes along a grid
-// dimension (N < 2^28). K of one chunk or below 16 (rows read in pieces of 8, 4,
-// 2 and 1 bytes): no split along K, 32x32 tiles of 2 x 2 waves until 64x128 tiles
-// fill the CUs: with waves split along K all but one are idle there
+// gemm_generic_kernel's tile (d.bm x d.bn) and waves (us, operands streamed
+// from HBM). 64x128 tiles (2 x 2 waves of 32x64) once they fill the CUs:
+// 4096x4096x4080 223 against 246 for 64x64 tiles and 368 for 32x32 ones,
+// 777x4096x1376 (416 tiles) 23.8 against 24.4 and 28.0, its rows unaligned
+// 30.2 against 35.3 and 49.1. Below that 32x32 tiles with two waves along K
+// (200x4096x1376 10.9 against 12.8 on 64x64 tiles), four where the tiles are
+// at most two per CU (64x4096x1376 6.3 against 7.7 with two, 575x512x560 5.8
+// against 6.5). Up to 32 rows, 16x16 tiles with eight waves while they are at
+// most two per CU (16x4096x1376 4.6 against 5.9 on 32x32 tiles, 32x2048x1001
+// 4.6 against 6.3), for more columns 16x32 tiles up to 16 rows (8x8192x5000
+// 13.7 against 15.2 on 16x16 tiles and 14.5 on 32x32) while their 512
+// work-items each stay below the 2^32 that a launch takes along a grid
+// dimension (N < 2^28). K of one chunk or below 16 (rows read in pieces of 8,
+// 4, 2 and 1 bytes): no split along K, 32x32 tiles of 2 x 2 waves until 64x128
+// tiles fill the CUs: with waves split along K all but one are idle there
 // (551x2171x20 10.1 us so, 6.2 unsplit; 4000x4000x12 123 and 25.5).
 void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int64_t block_k, int cus) {
   auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -3917,12 +3924,12 @@ void resolve_generic(Dispatch& d, int64_t M, int64_t N, int64_t K, int64_t block
 }
 
 // Ragged K on 16-byte aligned rows takes gemm_pipe128_kernel's fp16 form where
-// its tiles cover three quarters of the CUs: 777x4096x1376 (224 tiles) 19.3 us
-// against 22.8 on gemm_generic_kernel, 4096x4096x4080 181 against 211,
-// 300x8192x528 (192 tiles) 10.9 against 13.3; with half of the CUs
-// (400x4096x1376, 128 tiles) 18.4 against 16.5. Up to 64 rows most of a tile
-// is idle: 16x65536x528 21.5 against 16.2, 64x32768x1008 17.3 against 16.5
-// (100x28672x1008 16.7 against 18.7). Row counts that gemm_generic_kernel's
+// its tiles cover three quarters of the CUs: 777x4096x1376 (224 tiles) 20.0 us
+// against 23.8 on gemm_generic_kernel, 4096x4096x4080 214 against 223,
+// 300x8192x528 (192 tiles) 12.1 against 13.3; with half of the CUs
+// (400x4096x1376, 128 tiles) 19.6 against 17.6. Up to 64 rows most of a tile
+// is idle: 16x65536x528 24.8 against 18.4, 64x32768x1008 20.1 against 19.1
+// (100x28672x1008 20.3 against 21.1). Row counts that gemm_generic_kernel's
 // grid does not take are refused there, and 2^23 tiles or more, whose launch
 // would have 2^32 work-items in one dimension, run on its two-dimensional grid.
 bool ragged_pipe128(int64_t M, int64_t t128, int cus) {
