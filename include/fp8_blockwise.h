@@ -109,6 +109,8 @@ int fp8b_act_quant_typed(const void* x, int64_t ldx, int x_dtype,
  * multiples of 16 take the fp8 MFMA path; any other positive block sizes, K
  * and alignments take slower kernels with the same semantics (fp16 MFMAs on
  * the converted codes, fp32 sums).
+ * The fp8 MFMA path multiplies each sum by the product As * Bs, which has to
+ * be a normal fp32 number; the others multiply by As, then by Bs.
  * workspace may be NULL when fp8b_gemm_workspace_size() returns 0 for the
  * same arguments; otherwise it must hold at least that many bytes.
  */
