@@ -221,7 +221,7 @@ def main():
     args = parse()
     if args.gpus != 1:
         print(f"bench.py measures one GPU only: --gpus {args.gpus} is not supported "
-              "(every GPU box in this build has a single MI355X; across GPUs act-quant "
+              "(across GPUs act-quant "
               "would shard by rows and the GEMM by output columns, or by K with one "
               "all-reduce of the output; that path is not built)", file=sys.stderr)
         sys.exit(2)

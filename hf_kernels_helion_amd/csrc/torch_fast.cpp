@@ -1,16 +1,15 @@
 // Direct Python bindings of the hot ops (module _fp8_fast), for eager calls.
 //
 // A torch.ops call parses its arguments against the schema, boxes them and
-// goes through the dispatcher: ~2 us of host time per call on the MI355X
-// boxes' hosts, more than a small GEMM or act-quant kernel runs. These
-// bindings call the same C++ op functions (torch_ops.h) without it. Each
-// returns None, so that the Python wrapper takes the torch.ops route, unless
-// the call is a plain eager one: every tensor argument exactly a dense
-// torch.Tensor (no subclass such as FakeTensor, no meta tensor, no negated
-// view), none requiring grad, and no
-// TorchDispatchMode, torch-function mode, functorch transform or TorchScript
-// trace active (a trace would record the functions' at::empty and miss the
-// kernel that fills it). Results and errors are those of the torch.ops route
+// goes through the dispatcher: ~2 us of host time per call beside an MI355X,
+// more than a small GEMM or act-quant kernel runs. These bindings call the
+// same C++ op functions (torch_ops.h) without it. Each returns None, so that
+// the Python wrapper takes the torch.ops route, unless the call is a plain
+// eager one: every tensor argument exactly a dense torch.Tensor (no subclass
+// such as FakeTensor, no meta tensor, no negated view), none requiring grad,
+// and no TorchDispatchMode, torch-function mode, functorch transform or
+// TorchScript trace active (a trace would record the functions' at::empty and
+// miss the kernel that fills it). Results and errors are those of the torch.ops route
 // (same functions).
 #include <torch/extension.h>
 

@@ -3,7 +3,7 @@
 Restates finegrained-fp8-helion/bench.py:11-14 with the weight scales
 expanded over both N and K (the finegrained layout Bs[N/bn, K/bk]), plus the
 CPU act-quant for configurations that quantise activations in-op. bench.py
-times these on the GPU box's host cores as the reported CPU baseline; tests
+times these on the GPU host's cores as the reported CPU baseline; tests
 use them as a second, independent formulation.
 """
 from __future__ import annotations
